@@ -151,20 +151,31 @@ int plan_attention(int B, int H, int G, int D, int dma_kv, AttnPlan* plan) {
   plan->dma = false;
   plan->lds_bytes = lds;
   plan->rows = false;
+  plan->mfma = false;
   plan->rows_nkv = plan->rows_wpk = plan->rows_groups = 0;
   if (dma_kv <= 0) return SLMT_OK;
 
-  // Whole-row kernel first: it covers head_dim 64 and 128 with 4 or 8 query
-  // heads per KV head.  The workspace is sized for the larger of its grid and the
-  // other plans' (W_ws).
-  int nkv, wpk, rgroups;
+  // Whole-row kernels first: the matrix-core one covers up to 8 query heads per
+  // KV head at every head_dim, the vector-ALU one 4 or 8 at head_dim 64 and 128.
+  // The workspace is sized for the largest grid of any plan (W_ws).
+  int nkv, wpk, rgroups, w_rows = 0;
   if (rows_shape(H, G, D, dma_kv, &nkv, &wpk, &rgroups)) {
     plan->rows = true;
     plan->rows_nkv = nkv;
     plan->rows_wpk = wpk;
     plan->rows_groups = rgroups;
-    plan->W_ws = std::max(plan->W_ws, rows_max_workgroups(D, nkv, wpk, rgroups, cus));
+    w_rows = rows_max_workgroups(D, nkv, wpk, rgroups, cus);
   }
+  if (mfma_shape(H, G, D, dma_kv, &nkv, &wpk, &rgroups)) {
+    w_rows = std::max(w_rows, mfma_max_workgroups(D, nkv, wpk, rgroups, cus));
+    if (mfma_enabled()) {
+      plan->rows = plan->mfma = true;
+      plan->rows_nkv = nkv;
+      plan->rows_wpk = wpk;
+      plan->rows_groups = rgroups;
+    }
+  }
+  plan->W_ws = std::max(plan->W_ws, w_rows);
 
   // Direct-load plan: every wave's 4 heads share one KV head (G % 4 == 0) and
   // cache rows are a multiple of 16 bytes (an even number of KV heads), so a
@@ -181,8 +192,13 @@ int plan_attention(int B, int H, int G, int D, int dma_kv, AttnPlan* plan) {
   plan->dma = true;
   plan->lds_bytes = (size_t)geo.total;
   if (plan->W > plan->W_ws) plan->W_ws = plan->W;
-  if (plan->rows) plan->W_ws = std::max(plan->W_ws, rows_max_workgroups(D, nkv, wpk, rgroups, cus));
   return SLMT_OK;
+}
+
+// Head groups the limit on (sequence, head group) pairs counts.  The whole-row
+// kernels use no counters; the limit stays where each shape has always had it.
+static int counter_groups(const AttnPlan& pl, int G, int D) {
+  return pl.rows && D != 80 && (G == 4 || G == 8) ? std::max(pl.groups, pl.rows_groups) : pl.groups;
 }
 
 int64_t attention_workspace_bytes(int B, int H, int KV, int D) {
@@ -192,7 +208,7 @@ int64_t attention_workspace_bytes(int B, int H, int KV, int D) {
   }
   AttnPlan pl;
   if (plan_attention(B, H, H / KV, D, KV, &pl) != SLMT_OK) return -1;
-  if ((int64_t)std::max(pl.groups, pl.rows_groups) * B > kCounterCap) {
+  if ((int64_t)counter_groups(pl, H / KV, D) * B > kCounterCap) {
     fail(SLMT_ERR_UNSUPPORTED, "attention: more than 2^20 (sequence, head group) pairs in one call");
     return -1;
   }
@@ -210,8 +226,7 @@ int launch_attention(int mode, int D, AttnParams& p, void* workspace, int64_t ws
   AttnPlan pl;
   int rc = plan_attention(p.B, p.H, p.G, D, dma_ok ? p.cache_kv : 0, &pl);
   if (rc != SLMT_OK) return rc;
-  const int groups = pl.rows ? std::max(pl.groups, pl.rows_groups) : pl.groups;
-  if ((int64_t)groups * p.B > kCounterCap)
+  if ((int64_t)counter_groups(pl, p.G, D) * p.B > kCounterCap)
     return fail(SLMT_ERR_UNSUPPORTED, "attention: more than 2^20 (sequence, head group) pairs in one call");
   const WsLayout lay = ws_layout(pl, p.B, p.H, D);
   if (workspace == nullptr || ws_bytes < lay.total)
@@ -227,7 +242,7 @@ int launch_attention(int mode, int D, AttnParams& p, void* workspace, int64_t ws
   if (p.min_tiles <= 0) p.min_tiles = 4;
   if (mode == SRC_PAGED && pl.rows) {
     p.W = pl.W_ws;   // the kernel lowers it to the workgroups the CUs hold (no counters used)
-    if (mfma_rows_enabled(D, pl.rows_nkv, pl.rows_wpk))
+    if (pl.mfma)
       return launch_attention_mfma(D, pl.rows_nkv, pl.rows_wpk, pl.rows_groups, p, stream);
     return launch_attention_rows(D, pl.rows_nkv, pl.rows_wpk, pl.rows_groups, p, stream);
   }

@@ -229,6 +229,22 @@ __device__ __forceinline__ int seq_len_lane(const AttnParams& p, int b) {
 template <int TT>
 __device__ __forceinline__ int tiles_of(int L) { return (L + TT - 1) / TT; }
 
+// Workgroups that share T tiles: at least min_tiles tiles each; min_tiles 0 (the
+// matrix-core kernel, 64-token tiles) means 1, 2 or 4 tiles, so that a sequence of
+// the average length is cut into about 16 pieces, which the merge reads in one
+// batch.  With 4 tiles always, 16 requests of 200-4096 tokens at 12 q / 2 KV heads
+// left half of the chip idle.
+__device__ __forceinline__ int effective_workgroups(const AttnParams& p, int T) {
+  int n;
+  if (p.min_tiles > 0) {
+    n = (T + p.min_tiles - 1) / p.min_tiles;
+  } else {
+    const int sh = T < 24 * p.B ? 0 : T < 48 * p.B ? 1 : 2;
+    n = (T + (1 << sh) - 1) >> sh;
+  }
+  return max(1, min(p.W, n));
+}
+
 // First tile of workgroup w when T tiles are split over Weff workgroups.
 __device__ __forceinline__ int range_start(int w, int T, int Weff) {
   return (int)(((long long)w * T) / Weff);
@@ -344,7 +360,7 @@ __device__ bool schedule_range(const AttnParams& p, int* misc, int h0, int h1, T
     my_excl = v - mysum + misc[wave];
     r.T = uniform(misc[nwaves]);
   }
-  r.Weff = max(1, min(p.W, (r.T + p.min_tiles - 1) / p.min_tiles));
+  r.Weff = effective_workgroups(p, r.T);
   const int wg = blockIdx.x;
   if (wg >= r.Weff) return false;
   if (ZERO || r.T == 0) zero_empty<D>(p, h0, h1, r.Weff);
@@ -529,7 +545,7 @@ __device__ void split_merge(const AttnParams& p) {
     return;
   }
   const int Tb = tiles_of<TT>(L);
-  const int Weff = max(1, min(p.W, (T + p.min_tiles - 1) / p.min_tiles));
+  const int Weff = effective_workgroups(p, T);
   const int w_first = range_owner(Pb, T, Weff), w_last = range_owner(Pb + Tb - 1, T, Weff);
   if (w_first == w_last) return;   // one workgroup wrote the output
   const int first_slot = (range_start(w_first, T, Weff) == Pb) ? 0 : 1;

@@ -1,5 +1,5 @@
-// Batched paged 4-bit decode attention on the matrix cores, head_dim 64 or 128
-// with 4 or 8 query heads per KV head (reference kernel it replaces:
+// Batched paged 4-bit decode attention on the matrix cores, head_dim 64, 80 or 128
+// with 1 to 8 query heads per KV head (reference kernel it replaces:
 // kv_dequant_decode_per_token_paged_kernel, kernels/kv_dequant_kernels.cuh:671-801,
 // batched over the whole decode step instead of launched per request).
 //
@@ -15,13 +15,29 @@
 // query heads (WPK waves per KV head); 64-token tiles are copied with 16-byte
 // direct loads into a 2-stage LDS ring two tiles ahead; work is split stream-K
 // over the concatenated tile list and split sequences are merged by merge_kernel.
-// At head_dim 128 with 8 query heads per KV head the two waves of a KV head
+// At head_dim 80 and 128 with 8 head slots per KV head the two waves of a KV head
 // split each tile's tokens instead (32 each, all 8 heads as two sets of B
 // columns), so the nibble unpacking of K and V is done once per token rather
 // than once per wave; the second wave's sums join the first's through LDS at
 // each segment end.  At head_dim 64 the split measured slower (the extra
 // softmax reductions and the join cost more than the unpacking saved) and the
 // two waves take 4 heads each over the whole tile.
+//
+// Query heads per KV head other than 4 and 8 take the next larger number of head
+// slots, and head_dim 80 the two-block layout of 128 with query limbs of 0 past
+// its dims: the products of an empty slot cost matrix-core time that is idle
+// anyway, while the bytes read, the unpacking and the softmax stay per token and
+// KV head.  Against the per-wave vector-ALU kernel, which served these shapes
+// before (its register-staged form for other than multiples of 4 heads), us per
+// call, lengths U[500, 8000] or U[500, 4000] (*), fp16 out:
+//   12 q / 2 KV heads, 128 dims, batch 128     286.8 -> 38.9
+//   14 q / 2 KV heads,  64 dims, batch 64 (*)   56.4 -> 18.3
+//   32 q / 32 KV heads, 128 dims, batch 16 (*) 247.7 -> 34.7
+//   32 q / 8 KV heads,  80 dims, batch 64       95.1 -> 44.2
+//    8 q / 8 KV heads,  80 dims, batch 64 (*)   99.3 -> 29.1
+// and against the 32-token vector-ALU whole-row kernel (4 heads, a KV head count
+// that only 2 divides): 24 q / 6 KV heads, batch 64, 66.7 -> 62.1 at 128 dims and
+// 45.4 -> 38.2 at 64.
 //
 // QK, exact: v_mfma_i32_16x16x64_i8.  The fp16 query of each head is scaled by a
 // power of two to a 31-bit integer Q (every fp16 value above 2^-21 of the head's
@@ -70,7 +86,7 @@ typedef __attribute__((address_space(3))) const uint64_t lds_u64;
 
 template <int D, int NKV, int WPK>
 struct Shape {
-  static_assert(D == 64 || D == 128, "head_dim 64 or 128");
+  static_assert(D == 64 || D == 80 || D == 128, "head_dim 64, 80 or 128");
   static_assert(NKV % 2 == 0, "sub-rows must be a whole number of 16-byte units");
   static constexpr int TT = 64;                 // tokens per tile
   static constexpr int SLOT = D + 8;            // bytes of one KV head in a cache row
@@ -86,8 +102,9 @@ struct Shape {
   static constexpr int NOPS = (WUNITS + 63) / 64;
   static constexpr int LAST = WUNITS - 64 * (NOPS - 1);   // lanes of the wave's last load
   static constexpr int RB = TT / 16;            // QK row blocks (16 tokens)
-  static constexpr int KB = D / 64;             // QK k-blocks (64 dims)
-  static constexpr int CB = D / 64;             // PV blocks of 32 V bytes
+  static constexpr int KB = D == 64 ? 1 : 2;    // QK k-blocks (64 dims; past head_dim the query limbs are 0)
+  static constexpr int CB = KB;                 // PV blocks of 32 V bytes
+  static constexpr int VCOLS = D / (4 * CB);    // lanes of a row group that hold V bytes (2 CB bytes each)
   static constexpr int TH = TT / 32;            // PV token halves
   static constexpr int STAGE = TT * RSTRIDE;
   static constexpr int QOFF = NS * STAGE;       // one 1 KB query slot per wave
@@ -101,10 +118,10 @@ struct Shape {
   static constexpr int SOFF = MOFF + 32 * 4;
   // Two waves per KV head split each tile's tokens and take all of the KV head's
   // 8 query heads; at a segment end the second wave hands its (m, l, PV sums)
-  // to the first through this buffer: per KV head 64 lanes x D/4 floats + 3 x 8.
-  static constexpr int CBW = (D / 4) * 64 * 4 + 3 * 8 * 4;
+  // to the first through this buffer: per KV head 64 lanes x 16 CB floats + 3 x 8.
+  static constexpr int CBW = 16 * CB * 64 * 4 + 3 * 8 * 4;
   static constexpr int COFF = SOFF + STASH * 4;
-  static constexpr bool TS = WPK == 2 && D == 128;   // token split (see mfma_kernel)
+  static constexpr bool TS = WPK == 2 && D != 64;    // token split (see mfma_kernel)
   // Non-temporal tile loads, except with two KV heads per workgroup at head_dim
   // 64: there the halves of a cache row go to different workgroups, and the
   // 64-byte line that straddles them is read by both; with the default policy
@@ -125,7 +142,7 @@ constexpr float kRefMargin = 4.0f;
 
 // log2(e) / sqrt(D)
 template <int D>
-constexpr float kC = D == 128 ? 1.4426950408889634f / 11.313708498984761f : 1.4426950408889634f / 8.0f;
+constexpr float kC = 1.4426950408889634f / (D == 64 ? 8.0f : D == 80 ? 8.94427190999916f : 11.313708498984761f);
 
 // PV k-slot e (e < 8) of lane group g covers token ktok(g, e) of a 32-token
 // half: 8 m + 4 (g & 1) + 2 (g >> 1) + s for e = 2 m + s.  The rows that the
@@ -140,7 +157,9 @@ __device__ __forceinline__ int wpos(int t) {
   return 8 * g + 2 * (t >> 3) + (u & 1);
 }
 
-template <int D, int NKV, int WPK>
+// FULL: 4 WPK query heads per KV head, every head slot taken (a runtime count in
+// its place costs 1 % at 32 q / 8 KV heads, batch 64: registers and addresses).
+template <int D, int NKV, int WPK, bool FULL>
 __global__ void __launch_bounds__(NKV * WPK * 64) mfma_kernel(const AttnParams p) {
   using S = Shape<D, NKV, WPK>;
   constexpr int TT = S::TT, SLOT = S::SLOT, RB = S::RB, KB = S::KB, CB = S::CB, TH = S::TH;
@@ -161,10 +180,12 @@ __global__ void __launch_bounds__(NKV * WPK * 64) mfma_kernel(const AttnParams p
   const int wave = uniform(tid >> 6);
   const int group = blockIdx.y;
   const int wg = blockIdx.x;
-  const int h0 = group * 4 * S::WAVES, h1 = h0 + 4 * S::WAVES;   // the host checks H % (4 * WAVES) == 0
+  const int G = FULL ? 4 * WPK : p.G;                             // query heads per KV head, 1 .. 4 WPK
   const int kv_lo = group * NKV;
+  const int h0 = kv_lo * G, h1 = h0 + NKV * G;
   const int kvw = wave / WPK;                                     // the wave's KV head within the group
-  const int hw = h0 + 4 * wave;                                   // the wave's first query head
+  const int hk = (kv_lo + kvw) * G;                               // that KV head's first query head
+  const int hs = 4 * (wave % WPK);                                // the wave's first head slot of the KV head's 4 WPK
   const int half = TS ? (wave & 1) : 0;                           // token half (token split)
   int* misc = reinterpret_cast<int*>(smem + S::MOFF);
   uint8_t* const wscr = smem + S::WOFF + wave * S::WSZ;
@@ -197,8 +218,10 @@ __global__ void __launch_bounds__(NKV * WPK * 64) mfma_kernel(const AttnParams p
   // 64: lanes qp >= 8 re-read dims 8(qp - 8) ..); the slot holds (head h, dim d)
   // at byte 64 (d / 8) + 16 h + 2 (d % 8)
   const int qp = lane >> 2, qg = lane & 3;
-  const int qd = D == 128 ? qp : (qp & 7);
-  const uint32_t qoff = (uint32_t)(((hw + qg) * p.q_head_stride + qd * 8) * 2);
+  // (head slots past the KV head's G re-read its last head; their results are
+  // dropped.  head_dim 80: lanes qp >= 10 re-read dims 72 .., dropped in begin_set)
+  const int qd = D == 64 ? (qp & 7) : min(qp, D / 8 - 1);
+  const uint32_t qoff = (uint32_t)(((hk + (FULL ? hs + qg : min(hs + qg, G - 1))) * p.q_head_stride + qd * 8) * 2);
 
   // Tile descriptors, 64 tiles at a time, lane i for tile dchunk + i: the
   // address of this wave's first row and an info word
@@ -337,8 +360,10 @@ __global__ void __launch_bounds__(NKV * WPK * 64) mfma_kernel(const AttnParams p
         const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          qv[kb][8 * u + 2 * i] = h2f((uint16_t)(ws[i] & 0xffffu));
-          qv[kb][8 * u + 2 * i + 1] = h2f((uint16_t)(ws[i] >> 16));
+          // head_dim 80: dims 80 .. 127 of the second k-block are 0 whatever codes they meet
+          const bool in = D != 80 || kb == 0 || grp == 0;
+          qv[kb][8 * u + 2 * i] = in ? h2f((uint16_t)(ws[i] & 0xffffu)) : 0.f;
+          qv[kb][8 * u + 2 * i + 1] = in ? h2f((uint16_t)(ws[i] >> 16)) : 0.f;
         }
       }
     float amax = 0.f;
@@ -439,7 +464,7 @@ __global__ void __launch_bounds__(NKV * WPK * 64) mfma_kernel(const AttnParams p
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const uint8_t* src = Sb + (32 * th + ktok(grp, e)) * S::RSTRIDE + D / 2;
-        if constexpr (D == 128) R.v[th][e] = *reinterpret_cast<const uint32_t*>(src + 4 * col);
+        if constexpr (D != 64) R.v[th][e] = *reinterpret_cast<const uint32_t*>(src + 4 * min(col, S::VCOLS - 1));
         else R.v[th][e] = *reinterpret_cast<const uint16_t*>(src + 2 * col);
       }
   };
@@ -649,12 +674,13 @@ __global__ void __launch_bounds__(NKV * WPK * 64) mfma_kernel(const AttnParams p
     float lt = for_pv_lane_set(lh);
     float vt = for_pv_lane_set(vh);
     float mt = for_pv_lane_set(mh);
-    const int h = hw + (col & (HPW - 1));   // lanes col >= HPW hold no output
+    // the lane's head (lanes col >= HPW and head slots past the KV head's G hold no output)
+    const int h = hk + (TS ? 0 : hs) + (col & (HPW - 1));
     if constexpr (TS) {
       // The second wave of the pair hands its sums to the first, which scales
       // both by exp2(m - max) and stores the 8 heads; the second stores nothing.
       float* const cb = reinterpret_cast<float*>(smem + S::COFF + kvw * S::CBW);
-      float* const cml = cb + (D / 4) * 64;
+      float* const cml = cb + 16 * CB * 64;
       if (half == 1) {
 #pragma unroll
         for (int c = 0; c < CB; ++c)
@@ -722,12 +748,13 @@ __global__ void __launch_bounds__(NKV * WPK * 64) mfma_kernel(const AttnParams p
   };
   auto flush = [&]() __attribute__((always_inline)) {
     if (pk == 0) return;
-    if (col < HPW) {
+    if (col < HPW && (FULL || (TS ? 0 : hs) + (col & (HPW - 1)) < G)) {
 #pragma unroll
       for (int c = 0; c < CB; ++c)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int d = (D == 128 ? 8 : 4) * (4 * grp + r) + 4 * c;
+          if (4 * grp + r >= S::VCOLS) continue;
+          const int d = 4 * CB * (4 * grp + r) + 4 * c;
           const float* o = ov[c][r];
           if (pk == 1) {
             if (p.out_f16) {
@@ -878,14 +905,15 @@ static const char* kernel_name() {
 template <int D, int NKV, int WPK>
 static int launch(AttnParams p, int groups, hipStream_t stream) {
   using S = Shape<D, NKV, WPK>;
-  auto kern = mfma_kernel<D, NKV, WPK>;
+  auto kern = p.G == 4 * WPK ? mfma_kernel<D, NKV, WPK, true> : mfma_kernel<D, NKV, WPK, false>;
   const int per_cu = blocks_per_cu(reinterpret_cast<const void*>(kern), S::THREADS, S::LDS);
   const int cus = device_cu_count();
   int W = std::max(1, cus * std::max(1, per_cu) / groups);
   if (W > p.W) W = p.W;          // the workspace holds partials for p.W workgroups
   p.W = W;
   p.nthreads = S::THREADS;
-  p.heads_per_group = 4 * S::WAVES;
+  p.heads_per_group = NKV * p.G;
+  p.min_tiles = 0;               // by the tiles per sequence (effective_workgroups)
   hipEvent_t ev0, ev1;
   if (kernel_timing_events(&ev0, &ev1, kernel_name<D, NKV, WPK>()))
     hipExtLaunchKernelGGL(kern, dim3(W, groups), dim3(S::THREADS), S::LDS, stream, ev0, ev1, 0, p);
@@ -902,19 +930,54 @@ static int launch(AttnParams p, int groups, hipStream_t stream) {
 
 }  // namespace mrows
 
-// The matrix-core kernel serves whole-row shapes whose 64-token tile splits
-// into whole blocks per wave (4 or 8 waves per workgroup).  SLMT_PAGED_DECODE=valu
-// selects the vector-ALU whole-row kernel instead.
-bool mfma_rows_enabled(int D, int nkv, int wpk) {
-  const int waves = nkv * wpk;
-  if ((D != 64 && D != 128) || (waves != 4 && waves != 8)) return false;
+bool mfma_enabled() {
   const char* e = std::getenv("SLMT_PAGED_DECODE");
   return !(e && std::strcmp(e, "valu") == 0);
 }
 
-#define SLMT_MROWS_CONFIGS(X) \
-  X(128, 8, 1) X(128, 4, 1) X(128, 4, 2) X(128, 2, 2) X(64, 8, 1) X(64, 4, 1) X(64, 4, 2) X(64, 2, 2)
+#define SLMT_MROWS_CONFIGS(X)                                                       \
+  X(128, 8, 1) X(128, 4, 1) X(128, 4, 2) X(128, 2, 2) X(80, 8, 1) X(80, 4, 1) X(80, 4, 2) X(80, 2, 2) \
+  X(64, 8, 1) X(64, 4, 1) X(64, 2, 2)
 #define SLMT_MROWS_KEY(d, a, b) ((d) * 100 + (a) * 10 + (b))
+
+// A workgroup takes 4 or 8 waves (a 64-token tile then splits into whole blocks
+// per wave), so KV heads in twos at least and an even number of them (cache rows
+// and their parts are then whole 16-byte units).  Up to 4 query heads per KV head
+// are one wave's four head slots, 5 to 8 take two waves; slots past the KV
+// head's heads repeat its last head and are dropped.  A KV head count that only
+// 2 divides takes two waves per KV head for any number of heads.
+bool mfma_shape(int H, int G, int D, int cache_kv, int* nkv, int* wpk, int* groups) {
+  if ((D != 64 && D != 80 && D != 128) || G < 1 || G > 8 || H % G != 0) return false;
+  const int KV = H / G;
+  if (cache_kv != KV || KV % 2 != 0) return false;
+  int n, w = G <= 4 ? 1 : 2;
+  // Two waves per KV head: at head_dim 64 two KV heads per workgroup (4 waves,
+  // three workgroups per CU) keep more independent waves on each SIMD than
+  // four (8 waves, one workgroup per CU by registers); at 128 the reverse
+  // measured faster.
+  if (w == 1) n = KV % 8 == 0 ? 8 : KV % 4 == 0 ? 4 : 2;
+  else n = D != 64 && KV % 4 == 0 ? 4 : 2;
+  if (n == 2) w = 2;
+  *nkv = n;
+  *wpk = w;
+  *groups = KV / n;
+  return true;
+}
+
+// Workgroups per head group the kernel may use (its workspace bound): at most
+// 8 waves per CU at head_dim 80 and 128 (up to 256 VGPRs each), 12 at 64, and
+// the ring's LDS.
+int mfma_max_workgroups(int D, int nkv, int wpk, int groups, int cus) {
+  size_t lds = 0;
+  switch (SLMT_MROWS_KEY(D, nkv, wpk)) {
+#define SLMT_MROWS_LDS(d, a, b) case SLMT_MROWS_KEY(d, a, b): lds = mrows::Shape<d, a, b>::LDS; break;
+    SLMT_MROWS_CONFIGS(SLMT_MROWS_LDS)
+#undef SLMT_MROWS_LDS
+    default: return 1;
+  }
+  const int per_cu = std::max(1, std::min((D == 64 ? 12 : 8) / (nkv * wpk), (int)((160 * 1024) / lds)));
+  return std::max(1, cus * per_cu / groups);
+}
 
 int launch_attention_mfma(int D, int nkv, int wpk, int groups, const AttnParams& p, hipStream_t stream) {
   switch (SLMT_MROWS_KEY(D, nkv, wpk)) {

@@ -235,7 +235,7 @@ struct AttnPlan {
   size_t lds_bytes;
   // whole-row kernel (head_dim 128, 4 or 8 query heads per KV head): KV heads
   // and waves per KV head of a workgroup, head groups
-  bool rows;
+  bool rows, mfma;   // mfma: the matrix-core kernel of the two
   int rows_nkv, rows_wpk, rows_groups;
 };
 
@@ -257,9 +257,12 @@ bool kernel_timing_events(hipEvent_t* start, hipEvent_t* stop, const char* kerne
 const char* kernel_timing_kernel();           // slmt_kernel_timing_kernel
 int set_kernel_timing(bool enable);            // slmt_kernel_timing
 int read_kernel_timing(float* us, int max_n);  // slmt_kernel_timing_read
-// Matrix-core variant of the whole-row kernel (attention_mfma.hip): whether it
-// serves a whole-row shape (SLMT_PAGED_DECODE=valu turns it off), and its launch.
-bool mfma_rows_enabled(int D, int nkv, int wpk);
+// Matrix-core whole-row kernel (attention_mfma.hip): whether it may be used
+// (SLMT_PAGED_DECODE=valu turns it off), its shape for a request (false if it
+// does not apply), the workgroups per head group it may use, and its launch.
+bool mfma_enabled();
+bool mfma_shape(int H, int G, int D, int cache_kv, int* nkv, int* wpk, int* groups);
+int mfma_max_workgroups(int D, int nkv, int wpk, int groups, int cus);
 int launch_attention_mfma(int D, int nkv, int wpk, int groups, const AttnParams& p, hipStream_t stream);
 int64_t attention_workspace_bytes(int B, int H, int KV, int D);
 

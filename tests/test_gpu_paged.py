@@ -258,3 +258,48 @@ def test_one_long_sequence_over_every_workgroup(H, KV, D, paged_kernel):
     merge combines all of them."""
     case = make_paged_case(seed=H + D, B=1, H=H, KV=KV, D=D, lens=[40000], dist="t3")
     assert_close(_run_batched(case), paged_reference(case), what=f"one 40K sequence H={H} D={D}")
+
+
+# Lengths around a tile's 64 tokens, its halves and the pieces of one sequence.
+_EDGES = [1, 15, 17, 31, 32, 33, 63, 64, 65, 700, 0, 1600]
+
+
+@pytest.mark.parametrize("H,KV,D", [(8, 8, 80), (16, 4, 80), (12, 2, 80), (32, 4, 80), (6, 2, 80), (20, 4, 128),
+                                    (12, 2, 128), (14, 2, 64), (24, 8, 64), (16, 8, 128), (4, 4, 64), (2, 2, 128),
+                                    (10, 2, 64), (6, 6, 128), (24, 6, 64)])
+def test_paged_partial_head_slots(H, KV, D, paged_kernel):
+    """1 to 8 query heads per KV head at each head_dim: head slots that no head
+    takes, KV head counts divided by 8, 4 or only 2, head_dim 80's half-empty
+    second block of dims; both table widths and output types."""
+    case = make_paged_case(seed=H * 17 + KV + D, B=len(_EDGES), H=H, KV=KV, D=D, block_size=32, lens=_EDGES)
+    ref = paged_reference(case)
+    got = _run_batched(case)
+    assert_close(got, ref, what=f"H={H} KV={KV} D={D}")
+    assert np.all(got[10] == 0.0)
+    assert_close(_run_batched(case, torch.float16, torch.int64), ref, what="fp16 out, int64 tables")
+
+
+@pytest.mark.parametrize("H,KV,D", [(12, 2, 128), (6, 2, 80), (14, 2, 64)])
+def test_paged_partial_head_slots_keep_heads_apart(H, KV, D, paged_kernel):
+    """A NaN or infinite query makes its own head NaN and no other, strided q
+    and out, and stale bytes past a sequence's end stay out."""
+    case = make_paged_case(seed=H + D, B=3, H=H, KV=KV, D=D, lens=[70, 200, 31], extra_blocks=1)
+    used = [case.block_tables[b, :-(-int(n) // 16)] for b, n in enumerate(case.seq_lens)]
+    for b, n in enumerate(case.seq_lens.tolist()):
+        if n % 16:
+            case.kv_cache[int(used[b][-1]), n % 16:] = 0xFF
+    ref = paged_reference(case)
+    kd = _kd()
+    q = case.q.clone()
+    q[0, H - 1, D - 1] = float("nan")
+    q[2, 0, 3] = float("inf")
+    wide = torch.zeros((3, H + 2, D), dtype=torch.float16, device=DEV)
+    wide[:, 1:H + 1] = q.to(DEV)
+    out = torch.zeros((3, H + 1, D), dtype=torch.float32, device=DEV)
+    kd.kv_dequant_decode_paged_batched(wide[:, 1:H + 1], torch.from_numpy(case.kv_cache).to(DEV),
+                                       case.block_tables.to(DEV), case.seq_lens.to(DEV), 16, KV, out=out[:, :H])
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert np.isnan(got[0, H - 1]).all() and np.isnan(got[2, 0]).all() and np.all(got[:, H] == 0.0)
+    got[0, H - 1], got[2, 0] = ref[0, H - 1], ref[2, 0]
+    assert_close(got[:, :H], ref, what=f"H={H} D={D}")
