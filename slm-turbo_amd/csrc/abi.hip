@@ -342,33 +342,13 @@ int slmt_prefill_per_channel(const void* q, const void* k_packed, const void* k_
   if (rc != SLMT_OK) return rc;
   if (num_queries < 0) return fail(SLMT_ERR_INVALID, "kv_dequant_prefill: M must be >= 0");
   if (num_queries == 0) return SLMT_OK;
-  if (prefill_mfma_supported(head_dim))
-    return launch_prefill_mfma(q, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero, num_heads,
-                               num_heads / num_kv_heads, num_queries, seq_len, head_dim, causal, use_quant, out,
-                               reinterpret_cast<hipStream_t>(stream));
-  rc = check_workspace(ph, num_queries, num_heads, num_kv_heads, head_dim, workspace, workspace_bytes);
-  if (rc != SLMT_OK) return rc;
-  AttnParams p = blank_params();
-  p.q = reinterpret_cast<const uint16_t*>(q);
-  p.q_seq_stride = head_dim;                          // query row m
-  p.q_head_stride = (int64_t)num_queries * head_dim;  // [H, M, D]
-  p.kp = reinterpret_cast<const uint8_t*>(k_packed);
-  p.vp = reinterpret_cast<const uint8_t*>(v_packed);
-  p.kr0 = reinterpret_cast<const uint16_t*>(k_scale);
-  p.kr1 = reinterpret_cast<const uint16_t*>(k_zero);
-  p.vr0 = reinterpret_cast<const uint16_t*>(v_scale);
-  p.vr1 = reinterpret_cast<const uint16_t*>(v_zero);
-  p.use_quant = use_quant ? 1 : 0;
-  p.s_rows = seq_len;
-  p.fixed_len = seq_len;
-  p.causal_rows = causal ? 1 : 0;
-  p.B = num_queries;
-  p.H = num_heads;
-  p.G = num_heads / num_kv_heads;
-  p.out = out;
-  p.out_seq_stride = head_dim;
-  p.out_head_stride = (int64_t)num_queries * head_dim;
-  return launch_attention(SRC_CHANNEL, head_dim, p, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
+  if (head_dim == 80) {   // its documented argument, though the kernel uses none of it
+    rc = check_workspace(ph, num_queries, num_heads, num_kv_heads, head_dim, workspace, workspace_bytes);
+    if (rc != SLMT_OK) return rc;
+  }
+  return launch_prefill_mfma(q, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero, num_heads,
+                             num_heads / num_kv_heads, num_queries, seq_len, head_dim, causal, use_quant, out,
+                             reinterpret_cast<hipStream_t>(stream));
 }
 
 int slmt_kernel_timing(int enable) {

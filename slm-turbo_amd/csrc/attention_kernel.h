@@ -5,8 +5,8 @@
 //   SRC_PAGED   paged per-token min/step cache [nb, bs, KV, D+8]
 //               (kernels/kv_dequant_kernels.cuh:671-801, batched here)
 //   SRC_TOKEN   contiguous per-token buffers (kernels/kv_dequant_kernels.cuh:528-655)
-//   SRC_CHANNEL contiguous per-channel buffers, decode and causal prefill
-//               (kernels/kv_dequant_kernels.cuh:113-275, 293-502)
+//   SRC_CHANNEL contiguous per-channel buffers, decode
+//               (kernels/kv_dequant_kernels.cuh:113-275)
 //
 // Design (GEMV-shaped and bandwidth-bound; no MFMA):
 // * Work split: the tokens of all sequences are cut into tiles (32 tokens on
@@ -217,13 +217,13 @@ __device__ __forceinline__ int64_t sload_i64(const void* base, int64_t idx) {
 // Length of sequence b; `b` must be wave-uniform (scalar load).
 __device__ __forceinline__ int seq_len_of(const AttnParams& p, int b) {
   if (b >= p.B) return 0;
-  int L = p.seq_lens ? sload_i32(p.seq_lens, b) : (p.causal_rows ? min(p.fixed_len, b + 1) : p.fixed_len);
+  int L = p.seq_lens ? sload_i32(p.seq_lens, b) : p.fixed_len;
   return L < 0 ? 0 : L;
 }
 // Same for a per-lane b (vector load).
 __device__ __forceinline__ int seq_len_lane(const AttnParams& p, int b) {
   if (b >= p.B) return 0;
-  int L = p.seq_lens ? p.seq_lens[b] : (p.causal_rows ? min(p.fixed_len, b + 1) : p.fixed_len);
+  int L = p.seq_lens ? p.seq_lens[b] : p.fixed_len;
   return L < 0 ? 0 : L;
 }
 template <int TT>

@@ -1,5 +1,5 @@
-// Per-channel 4-bit prefill attention on the matrix cores (gfx950 MFMA), head_dim 64
-// and 128 (reference kernel it replaces: kv_dequant_prefill_kernel,
+// Per-channel 4-bit prefill attention on the matrix cores (gfx950 MFMA), head_dim 64,
+// 80 and 128 (reference kernel it replaces: kv_dequant_prefill_kernel,
 // kernels/kv_dequant_kernels.cuh:293-502).
 //
 // Prefill is GEMM-shaped (every key meets up to 64 query rows of a tile), so
@@ -42,6 +42,14 @@
 // reads are issued before the first QK product and all V^T operand reads
 // before the softmax, so LDS latency hides behind the products and the
 // exponentials instead of stalling each product.
+//
+// Head_dim 80 fills two and a half of QK's 32-dim blocks: the third block's upper
+// half is 0 in the query and in the staged K rows (written once).  Its codes past
+// dim 63 are staged evenly too, 2 bytes of K and 1 byte of V per key and thread,
+// so that no wave has more to convert than another.  Against the vector-ALU
+// kernel that took one query row at a time, us per causal prefill: 32 q / 8 KV
+// heads, 1000 tokens 480 -> 22, 4096 tokens 6277 -> 149; 8/8, 100 tokens 32.6 ->
+// 11.0 (the call's host time).  It is held to 168 VGPRs, three waves per SIMD.
 #include "slmt_internal.h"
 
 #include <type_traits>
@@ -75,7 +83,8 @@ struct Geo {
   // one such group, and only a row stride of 8 (mod 16) words keeps those 16
   // four-bank spans apart.  Rows of 16 bytes of padding (36 or 68 words) cost
   // 4 conflict cycles per read.
-  static constexpr int KROW = D * 2 + 32;
+  static constexpr int QB = (D + 31) / 32;  // 32-dim blocks of QK
+  static constexpr int KROW = QB * 64 + 32;
   // Bytes of a staged V^T row (keys in the order vpos gives, 32 bytes of
   // padding): the P.V operand of a lane is 16 contiguous bytes, one 16-byte read
   // (an 8-byte pair read moves half the bytes per cycle), conflict-free at a
@@ -86,6 +95,7 @@ struct Geo {
   static constexpr int LDS = 2 * STAGE;
   static constexpr int KW = D / 64;         // 8-byte K words per staging thread (K: 4 threads per key)
   static constexpr int VW = D / 64;         // V dwords per key per staging thread (V: 8 threads per key pair)
+  static constexpr bool X = D == 80;        // 16 dims more: 2 bytes of K, 1 of V per key and thread
 };
 
 __device__ __forceinline__ float hf(uint16_t h) { return h2f(h); }
@@ -108,7 +118,7 @@ __device__ __forceinline__ uint32_t nib_pair(uint32_t lo_all, uint32_t hi_all, i
 // Head_dim 64 is held to 128 VGPRs, four waves per SIMD (two 8-wave workgroups
 // per CU).
 template <int D, int HP>
-__global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 1))) prefill_kernel(const Params p) {
+__global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : D == 80 ? 3 : 1))) prefill_kernel(const Params p) {
   using GG = Geo<D>;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63, w = (tid >> 6) & 3;
@@ -128,27 +138,30 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
   // ---- the lane's query column, scaled per channel and by log2(e) / sqrt(D) (so
   // the scores come out as base-2 logits), split hi / lo (B operand of S^T)
   const float sc = 1.4426950408889634f * __builtin_amdgcn_rsqf((float)D);
-  half8 qh[D / 32], ql[D / 32];
+  constexpr int QB = GG::QB;
+  half8 qh[QB], ql[QB];
   {
     // The rulers are read whether or not use_quant is set (the pointers are
     // always valid), so that every load of the prologue is issued before the
     // first wait; under a per-element branch each load waited for the previous.
     const uint16_t* qrow = p.q + ((int64_t)h * p.M + mq) * D;
-    uint4 raw[D / 32];
-    uint16_t ksr[D / 32][8];
+    uint4 raw[QB];
+    uint16_t ksr[QB][8];
 #pragma unroll
-    for (int j = 0; j < D / 32; ++j) {
-      raw[j] = *reinterpret_cast<const uint4*>(qrow + 32 * j + 8 * grp);
+    for (int j = 0; j < QB; ++j) {
+      const int d0 = min(32 * j + 8 * grp, D - 8);   // head_dim 80, past its dims: re-read, zeroed below
+      raw[j] = *reinterpret_cast<const uint4*>(qrow + d0);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) ksr[j][e] = p.ks[(int64_t)kv * D + 32 * j + 8 * grp + e];
+      for (int e = 0; e < 8; ++e) ksr[j][e] = p.ks[(int64_t)kv * D + d0 + e];
     }
 #pragma unroll
-    for (int j = 0; j < D / 32; ++j) {
+    for (int j = 0; j < QB; ++j) {
       const uint32_t wds[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         float x = hf((uint16_t)(wds[e >> 1] >> (16 * (e & 1)))) * sc;
         x *= quant ? hf(ksr[j][e]) : 1.0f;
+        if (32 * j + 8 * grp >= D) x = 0.f;
         const _Float16 hi = (_Float16)x;
         qh[j][e] = hi;
         ql[j][e] = (_Float16)(x - (float)hi);
@@ -175,6 +188,12 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
   // (1024 + zero) of dims 2b and 2b + 1 of the thread's 8, one register per pair;
   // the packed subtractions below take one half of it for both lanes (op_sel)
   half2v vzc[GG::VW][4];
+  half2v vzx;                        // head_dim 80: of dims 64 + 2 vb and the next
+  if constexpr (GG::X) {
+    const uint16_t z0 = p.vz[(int64_t)kv * D + 64 + 2 * vb], z1 = p.vz[(int64_t)kv * D + 65 + 2 * vb];
+    vzx[0] = (_Float16)(1024.0f + zround(z0));
+    vzx[1] = (_Float16)(1024.0f + zround(z1));
+  }
   {
     uint16_t zr[GG::VW][8];
 #pragma unroll
@@ -199,7 +218,8 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
   // before it is computed, and written to LDS one tile before.
   uint2 kx[2][GG::KW];
   uint32_t vx[2][GG::VW][2];
-  const uint32_t koff0 = (uint32_t)(kk * (D / 2) + ku * (D / 8));
+  uint32_t kxx[2], vxx[2][2];        // head_dim 80: the codes past dim 63
+  const uint32_t koff0 = (uint32_t)(kk * (D / 2) + ku * 8 * GG::KW);
   const uint32_t voff0 = (uint32_t)(2 * vk * (D / 2) + 4 * vb);
   auto load = [&](int t, auto slot) {   // the tile's codes (keys past S re-read key S - 1)
     constexpr int sl = decltype(slot)::value;
@@ -213,10 +233,15 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
         vx[sl][r][0] = *reinterpret_cast<const uint32_t*>(vbase + (voff0 + off + 32 * r));
         vx[sl][r][1] = *reinterpret_cast<const uint32_t*>(vbase + (voff0 + off + D / 2 + 32 * r));
       }
+      if constexpr (GG::X) {
+        kxx[sl] = *reinterpret_cast<const uint16_t*>(kbase + (koff0 + off + 32 - 6 * ku));
+        vxx[sl][0] = vbase[voff0 + off + 32 - 3 * vb];
+        vxx[sl][1] = vbase[voff0 + off + D / 2 + 32 - 3 * vb];
+      }
       return;
     }
     const int key = min(t * BN + kk, p.S - 1);
-    const uint32_t ko = (uint32_t)(key * (D / 2) + ku * (D / 8));
+    const uint32_t ko = (uint32_t)(key * (D / 2) + ku * 8 * GG::KW);
 #pragma unroll
     for (int i = 0; i < GG::KW; ++i) kx[sl][i] = *reinterpret_cast<const uint2*>(kbase + (ko + 8 * i));
     const int k0 = min(t * BN + 2 * vk, p.S - 1), k1 = min(t * BN + 2 * vk + 1, p.S - 1);
@@ -225,13 +250,18 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
       vx[sl][r][0] = *reinterpret_cast<const uint32_t*>(vbase + (uint32_t)(k0 * (D / 2) + 4 * (vb + 8 * r)));
       vx[sl][r][1] = *reinterpret_cast<const uint32_t*>(vbase + (uint32_t)(k1 * (D / 2) + 4 * (vb + 8 * r)));
     }
+    if constexpr (GG::X) {
+      kxx[sl] = *reinterpret_cast<const uint16_t*>(kbase + (ko + 32 - 6 * ku));
+      vxx[sl][0] = vbase[(uint32_t)(k0 * (D / 2) + 32 + vb)];
+      vxx[sl][1] = vbase[(uint32_t)(k1 * (D / 2) + 32 + vb)];
+    }
   };
   auto store = [&](auto slot) {  // slot's codes -> fp16 (code - zero) in LDS stage `slot`
     constexpr int sl = decltype(slot)::value;
     if (!stager) return;
     uint8_t* Ks = smem + sl * GG::STAGE;
     uint8_t* Vs = Ks + GG::KBYTES;
-    uint32_t kw[D / 8];
+    uint32_t kw[8 * GG::KW];
 #pragma unroll
     for (int i = 0; i < GG::KW; ++i) {
       const uint32_t ws2[2] = {kx[sl][i].x, kx[sl][i].y};
@@ -245,9 +275,20 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
         }
       }
     }
-    uint4* kd = reinterpret_cast<uint4*>(Ks + kk * GG::KROW + ku * (D / 2));
+    uint4* kd = reinterpret_cast<uint4*>(Ks + kk * GG::KROW + ku * 32 * GG::KW);
 #pragma unroll
-    for (int i = 0; i < D / 32; ++i) kd[i] = make_uint4(kw[4 * i], kw[4 * i + 1], kw[4 * i + 2], kw[4 * i + 3]);
+    for (int i = 0; i < 2 * GG::KW; ++i) kd[i] = make_uint4(kw[4 * i], kw[4 * i + 1], kw[4 * i + 2], kw[4 * i + 3]);
+    if constexpr (GG::X) {
+      const uint32_t lo = kxx[sl] & 0x0F0Fu, hi = (kxx[sl] >> 4) & 0x0F0Fu;
+      *reinterpret_cast<uint2*>(Ks + kk * GG::KROW + 128 + 8 * ku) = make_uint2(nib_pair(lo, hi, 0, kzc), nib_pair(lo, hi, 1, kzc));
+      // the two keys' bytes: low nibbles are dim 64 + 2 vb, high nibbles the next
+      const uint32_t b2 = vxx[sl][0] | (vxx[sl][1] << 16);
+      const half2v ze = __builtin_shufflevector(vzx, vzx, 0, 0), zo = __builtin_shufflevector(vzx, vzx, 1, 1);
+      const half2v e = __builtin_bit_cast(half2v, (b2 & 0x000F000Fu) | 0x64006400u) - ze;
+      const half2v o = __builtin_bit_cast(half2v, ((b2 >> 4) & 0x000F000Fu) | 0x64006400u) - zo;
+      *reinterpret_cast<uint32_t*>(Vs + (64 + 2 * vb) * GG::VROW + vcol) = __builtin_bit_cast(uint32_t, e);
+      *reinterpret_cast<uint32_t*>(Vs + (65 + 2 * vb) * GG::VROW + vcol) = __builtin_bit_cast(uint32_t, o);
+    }
 #pragma unroll
     for (int r = 0; r < GG::VW; ++r) {
       const uint32_t lo0 = vx[sl][r][0] & 0x0F0F0F0Fu, hi0 = (vx[sl][r][0] >> 4) & 0x0F0F0F0Fu;
@@ -289,6 +330,12 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
   // are merged conservatively over paths that issue no loads, and with either
   // branch the staging store of tile t + 1 waited for the loads of tile t + 2
   // as well, which were issued in the same iteration.
+  if constexpr (GG::X) {             // the K rows' dims 80 .. 95, in both stages (row tid & 127)
+    if (tid < 128) {
+      uint4* z = reinterpret_cast<uint4*>(smem + (tid >> 6) * GG::STAGE + (tid & 63) * GG::KROW + 160);
+      z[0] = z[1] = make_uint4(0, 0, 0, 0);
+    }
+  }
   if (ntiles > 0) {
     load(0, S0{});
     load(min(1, ntiles - 1), S1{});
@@ -305,11 +352,11 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
     const uint8_t* Vs = Ks + GG::KBYTES;
     // S^T: keys 16 n + 4 grp + i of this tile against the lane's query
     // (all K operand reads are issued before the first product)
-    half8 ka[4][D / 32];
+    half8 ka[4][QB];
 #pragma unroll
     for (int n = 0; n < 4; ++n)
 #pragma unroll
-      for (int j = 0; j < D / 32; ++j)
+      for (int j = 0; j < QB; ++j)
         ka[n][j] = *reinterpret_cast<const half8*>(Ks + (16 * n + col) * GG::KROW + (32 * j + 8 * grp) * 2);
     __builtin_amdgcn_sched_barrier(0);
     floatx4 s[4];
@@ -318,7 +365,7 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
       s[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[n][0], qh[0], cinit, 0, 0, 0);
       s[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[n][0], ql[0], s[n], 0, 0, 0);
 #pragma unroll
-      for (int j = 1; j < D / 32; ++j) {
+      for (int j = 1; j < QB; ++j) {
         s[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[n][j], qh[j], s[n], 0, 0, 0);
         s[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[n][j], ql[j], s[n], 0, 0, 0);
       }
@@ -488,8 +535,6 @@ int launch(const Params& p, hipStream_t stream) {
 
 }  // namespace prefill
 
-bool prefill_mfma_supported(int D) { return D == 64 || D == 128; }
-
 int launch_prefill_mfma(const void* q, const void* kp, const void* ks, const void* kz, const void* vp, const void* vs,
                         const void* vz, int H, int G, int M, int S, int D, int causal, int use_quant, float* out,
                         hipStream_t stream) {
@@ -513,8 +558,9 @@ int launch_prefill_mfma(const void* q, const void* kp, const void* ks, const voi
   if (M <= 0) return SLMT_OK;
   if ((int64_t)p.qblocks * H > 0x7fffffff) return fail(SLMT_ERR_UNSUPPORTED, "prefill: too many query blocks");
   if (D == 64) return prefill::launch<64>(p, stream);
+  if (D == 80) return prefill::launch<80>(p, stream);
   if (D == 128) return prefill::launch<128>(p, stream);
-  return fail(SLMT_ERR_UNSUPPORTED, "prefill: the matrix-core kernel takes head_dim 64 or 128");
+  return fail(SLMT_ERR_INVALID, "kv_dequant_prefill: head_dim must be 64/80/128, got " + std::to_string(D));
 }
 
 }  // namespace slmt

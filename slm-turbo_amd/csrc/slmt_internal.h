@@ -208,10 +208,9 @@ struct AttnParams {
   const uint16_t* vr1;  // v_step  | v_zero
   int s_rows;           // S of the contiguous tensors
   int use_quant;
-  // sequences: L_b = seq_lens[b], or fixed_len, or min(fixed_len, b+1) (causal rows)
+  // sequences: L_b = seq_lens[b], or fixed_len
   const int32_t* seq_lens;
   int fixed_len;
-  int causal_rows;
   int B, H, G;           // G = H / num_kv_heads
   int heads_per_group;   // query heads per workgroup (multiple of 4)
   // output: element (b, h, d) at out + b*out_seq_stride + h*out_head_stride + d
@@ -280,9 +279,7 @@ int launch_decode_channel_split(const void* q, const void* kp, const void* ks, c
                                 const void* vs, const void* vz, int H, int G, int S, int D, int use_quant, float* out,
                                 void* workspace, int64_t ws_bytes, hipStream_t stream);
 
-// Per-channel prefill on the matrix cores (prefill_mfma.hip), head_dim 64 and 128;
-// no workspace.  q [H, M, D] fp16, codes [KV_t, S, D/2], rulers [KV_t, D].
-bool prefill_mfma_supported(int D);
+// Per-channel prefill on the matrix cores (prefill_mfma.hip); no workspace.  q [H, M, D] fp16, codes [KV_t, S, D/2], rulers [KV_t, D].
 int launch_prefill_mfma(const void* q, const void* kp, const void* ks, const void* kz, const void* vp, const void* vs,
                         const void* vz, int H, int G, int M, int S, int D, int causal, int use_quant, float* out,
                         hipStream_t stream);

@@ -223,6 +223,31 @@ def test_prefill_matrix_cores(H, KV, D, M, S, causal, outl, t3):
     assert_close(out, ref, what=f"prefill H={H} KV={KV} D={D} M={M} S={S}")
 
 
+# head_dim 80: one row, edges of the 64-row blocks and 64-key tiles, one and two
+# heads per workgroup (the second needs over 256 of them), raw codes, rulers that
+# are not 8-byte aligned.
+@pytest.mark.parametrize("H,KV,M,S,causal,quant,shift", [
+    (2, 2, 1, 1, True, True, 0), (4, 2, 63, 64, True, True, 1), (4, 2, 64, 65, False, True, 0),
+    (8, 2, 65, 63, True, False, 0), (6, 2, 200, 129, False, True, 1), (3, 3, 130, 500, True, True, 0),
+    (16, 2, 2100, 2100, True, True, 0)])
+def test_prefill_matrix_cores_head_dim_80(H, KV, M, S, causal, quant, shift):
+    q, t = _pf_inputs(H + 3 * M + S, H, KV, M, S, 80, outliers=M == 200)
+    dev = []
+    for x in t:
+        if x.dtype == torch.float16 and shift:
+            buf = torch.zeros(x.numel() + shift, dtype=torch.float16, device=DEV)
+            buf[shift:] = x.to(DEV).flatten()
+            dev.append(buf[shift:].view(x.shape))
+        else:
+            dev.append(x.to(DEV))
+    kw = dict(causal=causal, use_quant=quant, num_kv_heads=KV)
+    out = _kd().kv_dequant_prefill_attention(q.to(DEV), *dev, **kw)
+    torch.cuda.synchronize()
+    ref = oa.prefill_per_channel(q.numpy(), *[x.numpy() for x in t], causal=causal, use_quant=quant)
+    assert_close(out.cpu().numpy(), ref, what=f"prefill D=80 H={H} M={M} S={S}")
+    assert torch.equal(out, _kd().kv_dequant_prefill_attention(q.to(DEV), *dev, **kw))
+
+
 # Long causal prefills (up to 32 query blocks): one and two query heads per
 # workgroup, both head dims, outliers and Student-t K/V, and S > M with a partial
 # last block; a second call gives the same bits.
