@@ -88,6 +88,12 @@ int slmt_quantize_store(const void* key, int64_t key_token_stride,
 int slmt_quantize_per_channel(const void* x, int num_kv_heads, int seq_len, int head_dim,
                               void* packed, void* scale, void* zero, slmt_stream_t stream);
 
+/* K and V of one shape in the same launches (quantize_kv of the reference,
+ * kernels/benchmark/benchmark.py:69-74); each as slmt_quantize_per_channel. */
+int slmt_quantize_kv_per_channel(const void* k, const void* v, int num_kv_heads, int seq_len, int head_dim,
+                                 void* k_packed, void* k_scale, void* k_zero, void* v_packed, void* v_scale,
+                                 void* v_zero, slmt_stream_t stream);
+
 /*
  * Per-channel append with fixed rulers: the reference's quantize_tensor(x,
  * scale, zero_point) (host torch code, kernels/benchmark/benchmark.py:45-56),

@@ -182,19 +182,34 @@ int slmt_quantize_store(const void* key, int64_t key_token_stride, const void* v
                                num_kv_heads, head_dim, reinterpret_cast<hipStream_t>(stream));
 }
 
-int slmt_quantize_per_channel(const void* x, int num_kv_heads, int seq_len, int head_dim, void* packed,
-                              void* scale, void* zero, slmt_stream_t stream) {
+static int quantize_per_channel(int nt, const void* const* x, int num_kv_heads, int seq_len, int head_dim,
+                                void* const* packed, void* const* scale, void* const* zero, slmt_stream_t stream) {
   clear_error();
   if (!head_dim_ok(head_dim))
     return fail(SLMT_ERR_INVALID, "quantize: head_dim must be 64/80/128, got " + s(head_dim));
   if (num_kv_heads < 0 || seq_len <= 0)
     return fail(SLMT_ERR_INVALID, "quantize: need KV >= 0 and S >= 1 (got KV=" + s(num_kv_heads) + ", S=" + s(seq_len) + ")");
   if (num_kv_heads == 0) return SLMT_OK;
-  if (!x || !packed || !scale || !zero) return fail(SLMT_ERR_INVALID, "quantize: null pointer argument");
-  if (!aligned(x, 4) || !aligned(scale, 2) || !aligned(zero, 2))
-    return fail(SLMT_ERR_INVALID, "quantize: x must be 4-byte aligned");
-  return launch_quantize_per_channel(x, num_kv_heads, seq_len, head_dim, packed, scale, zero,
+  for (int i = 0; i < nt; ++i) {
+    if (!x[i] || !packed[i] || !scale[i] || !zero[i]) return fail(SLMT_ERR_INVALID, "quantize: null pointer argument");
+    if (!aligned(x[i], 4) || !aligned(scale[i], 2) || !aligned(zero[i], 2))
+      return fail(SLMT_ERR_INVALID, "quantize: x must be 4-byte aligned");
+  }
+  return launch_quantize_per_channel(nt, x, num_kv_heads, seq_len, head_dim, packed, scale, zero,
                                      reinterpret_cast<hipStream_t>(stream));
+}
+
+int slmt_quantize_per_channel(const void* x, int num_kv_heads, int seq_len, int head_dim, void* packed,
+                              void* scale, void* zero, slmt_stream_t stream) {
+  return quantize_per_channel(1, &x, num_kv_heads, seq_len, head_dim, &packed, &scale, &zero, stream);
+}
+
+int slmt_quantize_kv_per_channel(const void* k, const void* v, int num_kv_heads, int seq_len, int head_dim,
+                                 void* k_packed, void* k_scale, void* k_zero, void* v_packed, void* v_scale,
+                                 void* v_zero, slmt_stream_t stream) {
+  const void* x[2] = {k, v};
+  void *packed[2] = {k_packed, v_packed}, *scale[2] = {k_scale, v_scale}, *zero[2] = {k_zero, v_zero};
+  return quantize_per_channel(2, x, num_kv_heads, seq_len, head_dim, packed, scale, zero, stream);
 }
 
 int slmt_quantize_with_rulers(const void* x, int64_t x_head_stride, int64_t x_seq_stride, int num_kv_heads,

@@ -180,8 +180,9 @@ int launch_quantize_store(const void* key, int64_t key_stride, const void* value
 int launch_quantize_rulers(const void* x, int64_t x_head_stride, int64_t x_seq_stride, int KV, int S, int D,
                            const void* scale, const void* zero, void* packed, int64_t out_head_stride,
                            int64_t out_seq_stride, hipStream_t stream);
-int launch_quantize_per_channel(const void* x, int KV, int S, int D, void* packed,
-                                void* scale, void* zero, hipStream_t stream);
+// nt (1 or 2) tensors of one shape
+int launch_quantize_per_channel(int nt, const void* const* x, int KV, int S, int D, void* const* packed,
+                                void* const* scale, void* const* zero, hipStream_t stream);
 
 // Attention source layouts.
 enum SrcMode : int { SRC_PAGED = 0, SRC_TOKEN = 1, SRC_CHANNEL = 2 };

@@ -34,6 +34,7 @@ SIGNATURES = {
     "slmt_attention_workspace_bytes": (_i64, [_i32, _i32, _i32, _i32]),
     "slmt_quantize_store": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _i32, _p_i64, _i64, _i32, _i32, _vp]),
     "slmt_quantize_per_channel": (_i32, [_vp, _i32, _i32, _i32, _vp, _vp, _vp, _vp]),
+    "slmt_quantize_kv_per_channel": (_i32, [_vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "slmt_quantize_with_rulers": (_i32, [_vp, _i64, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _i64, _i64, _vp]),
     "slmt_decode_paged": (_i32, [_vp, _vp, _i64, _i32, _p_i64, _i32, _i32, _i32, _i32, _p_f32, _vp, _i64,
                                  _vp]),

@@ -526,7 +526,21 @@ def quantize_tensor(x, scale, zero_point, bits=4, out=None):
 
 def quantize_kv(k, v):
     """(k_packed, k_scale, k_zero, v_packed, v_scale, v_zero), like the
-    reference's quantize_kv (kernels/benchmark/benchmark.py:69-74)."""
+    reference's quantize_kv (kernels/benchmark/benchmark.py:69-74); K and V of one
+    shape go through the same launches."""
+    if k.dim() == 3 and k.shape == v.shape and k.dtype is v.dtype is torch.float16 and k.is_cuda \
+            and k.device == v.device and k.shape[1] >= 1 and k.shape[2] in _SUPPORTED_D:
+        KV, S, D = k.shape
+        lib = _load_native_extension()
+        dev = k.device
+        with _on_device(dev):
+            k, v = k.contiguous(), v.contiguous()
+            kp, vp = (torch.empty((KV, S, D // 2), dtype=torch.uint8, device=dev) for _ in range(2))
+            ks, kz, vs, vz = (torch.empty((KV, D), dtype=torch.float16, device=dev) for _ in range(4))
+            rc = lib.slmt_quantize_kv_per_channel(_ptr(k), _ptr(v), KV, S, D, _ptr(kp), _ptr(ks), _ptr(kz),
+                                                  _ptr(vp), _ptr(vs), _ptr(vz), _stream(dev))
+            _native.check(lib, rc)
+        return kp, ks, kz, vp, vs, vz
     kp, ks, kz = quantize_per_channel(k)
     vp, vs, vz = quantize_per_channel(v)
     return kp, ks, kz, vp, vs, vz

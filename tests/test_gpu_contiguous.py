@@ -360,3 +360,34 @@ def test_decode_per_channel_split_chunks(H, KV, D, S, outl):
         torch.cuda.synchronize()
         ref = oa.decode_per_channel(q.numpy(), *[x.numpy() for x in t])
         assert_close(out.cpu().numpy(), ref, what=f"H={H} KV={KV} D={D} S={S}")
+
+
+# The register kernel's thread and row counts (up to 4096 rows), the three launches
+# past it (chunks with remainders, several KV heads), inputs at odd multiples of 4
+# bytes, NaN and infinities, constant channels: each byte against the oracle, K and
+# V together as one by one.
+@pytest.mark.parametrize("KV,S,D", [(1, 1, 64), (2, 31, 80), (3, 32, 128), (2, 33, 64), (1, 511, 80), (2, 513, 128),
+                                    (2, 1025, 64), (1, 2049, 80), (2, 4096, 64), (2, 4097, 80), (3, 4999, 128),
+                                    (1, 9001, 64)])
+def test_quantize_kv_row_counts(KV, S, D):
+    g = torch.Generator().manual_seed(S + D)
+    k, v = torch.randn(KV, S, D, generator=g).half(), (3 * torch.randn(KV, S, D, generator=g)).half()
+    k[0, S // 2, 1] = float("nan")
+    k[0, S - 1, 2] = float("inf")
+    k[KV - 1, 0, 3] = -60000.0
+    v[:, :, 4] = 0.25
+    v[0, S - 1, D - 1] = 100.0
+    buf = torch.zeros(k.numel() + 2, dtype=torch.float16, device=DEV)
+    kd_ = buf[2:].view(k.shape)
+    kd_.copy_(k)
+    got = _kd().quantize_kv(kd_, v.to(DEV))
+    alone = _kd().quantize_per_channel(kd_)
+    torch.cuda.synchronize()
+    ref = oq.quantize_kv(k.numpy(), v.numpy())
+    for i, (a, b) in enumerate(zip(got, ref)):
+        if a.dtype == torch.uint8:
+            assert np.array_equal(a.cpu().numpy(), b), f"codes {i}: {int((a.cpu().numpy() != b).sum())} differ"
+        else:
+            _same_fp16(a.cpu().numpy(), b)
+    for a, b in zip(alone, got):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
