@@ -303,3 +303,36 @@ def test_paged_partial_head_slots_keep_heads_apart(H, KV, D, paged_kernel):
     assert np.isnan(got[0, H - 1]).all() and np.isnan(got[2, 0]).all() and np.all(got[:, H] == 0.0)
     got[0, H - 1], got[2, 0] = ref[0, H - 1], ref[2, 0]
     assert_close(got[:, :H], ref, what=f"H={H} D={D}")
+
+
+# Rows that leave a workgroup's last rows empty, rows that start on odd multiples of 4
+# bytes, constant rows, zeros of both signs, infinities and NaNs among numbers.
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 80, 128])
+@pytest.mark.parametrize("N,KV", [(1, 1), (5, 3), (33, 8)])
+def test_store_row_remainders_and_special_values(N, KV, D):
+    from oracle import quant as oq
+
+    kd = _kd()
+    g = torch.Generator().manual_seed(N * D)
+    x = torch.randn(2, N, KV, D, generator=g)
+    x[:, 0, 0] = 0.5
+    if N > 1:
+        x[:, 1] = torch.where(x[:, 1] > 0, 0.0, -0.0)
+        x[:, 2, 0, 3] = float("inf")
+        x[:, 2, 1, 4] = float("nan")
+        x[:, 3] *= 1e-6
+        x[:, 4] *= 2e4
+    x = x.half()
+    slots = torch.randperm(N + 7, generator=g)[:N]
+    slots[N // 2] = -1 if N > 1 else slots[0]
+    nb = (N + 7 + 15) // 16
+    ref = np.zeros((nb, 16, KV, D + 8), dtype=np.uint8)
+    oq.quantize_store(x[0].numpy(), x[1].numpy(), ref, slots.numpy(), 16)
+    cache = torch.zeros(ref.shape, dtype=torch.uint8, device="cuda:0")
+    wide = torch.zeros(2, N, KV * D + 2, dtype=torch.float16, device="cuda:0")
+    wide[:, :, 2:] = x.reshape(2, N, -1).to("cuda:0")
+    k, v = (wide[i, :, 2:].unflatten(1, (KV, D)) for i in range(2))
+    kd.kv_quantize_store(k, v, cache, slots.to("cuda:0"), 16)
+    torch.cuda.synchronize()
+    assert np.array_equal(cache.cpu().numpy(), ref)
