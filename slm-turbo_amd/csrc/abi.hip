@@ -310,9 +310,8 @@ int slmt_decode_per_channel(const void* q, const void* k_packed, const void* k_s
   rc = check_workspace(ph, 1, num_heads, num_kv_heads, head_dim, workspace, workspace_bytes);
   if (rc != SLMT_OK) return rc;
   // one short sequence: split over (KV head, key chunk) when the shape allows it
-  rc = launch_decode_channel_split(q, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero, num_heads,
-                                   num_heads / num_kv_heads, seq_len, head_dim, use_quant, out, workspace,
-                                   workspace_bytes, reinterpret_cast<hipStream_t>(stream));
+  rc = launch_decode_split(false, q, k_packed, v_packed, r, num_heads, num_heads / num_kv_heads, seq_len, head_dim,
+                           use_quant, out, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
   if (rc != SLMT_ERR_UNSUPPORTED) return rc;
   AttnParams p = blank_params();
   p.q = reinterpret_cast<const uint16_t*>(q);
@@ -333,6 +332,10 @@ int slmt_decode_per_channel(const void* q, const void* k_packed, const void* k_s
   p.out = out;
   p.out_seq_stride = (int64_t)num_heads * head_dim;
   p.out_head_stride = head_dim;
+  // one short sequence: split over (KV head, key chunk) when the shape allows it
+  rc = launch_decode_split(true, q, k_packed, v_packed, r, num_heads, num_heads / num_kv_heads, seq_len, head_dim, 1,
+                           out, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
+  if (rc != SLMT_ERR_UNSUPPORTED) return rc;
   return launch_attention(SRC_CHANNEL, head_dim, p, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
 }
 

@@ -1,7 +1,8 @@
-// Single-sequence per-channel 4-bit decode, split over (KV head, key chunk)
-// workgroups (reference kernel it replaces for head_dim 64 / 128 and up to 8
-// query heads per KV head: kv_dequant_decode_kernel,
-// kernels/kv_dequant_kernels.cuh:113-275).
+// Single-sequence 4-bit decode over contiguous per-channel or per-token buffers,
+// split over (KV head, key chunk) workgroups (reference kernels it replaces for up
+// to 8 query heads per KV head: kv_dequant_decode_kernel,
+// kernels/kv_dequant_kernels.cuh:113-275, and kv_dequant_decode_per_token_kernel,
+// :528-655).
 //
 // The reference's op-level decode is one query row over a short context (tens
 // of KB to a few MB of packed K/V), so the call is bound by latency, not by
@@ -9,8 +10,8 @@
 // and the work on it.  A single wave issues a vector instruction only every
 // ~8 cycles, so the per-wave work must be short: one workgroup of four waves
 // per (KV head kv, chunk of CT keys), each wave CT/4 keys:
-//   * the G query heads of kv, scaled per channel (q'_d = q_d * k_scale_d), go
-//     to LDS;
+//   * the G query heads of kv, scaled per channel (q'_d = q_d * k_scale_d; per
+//     token: as they are), go to LDS;
 //   * QK, 16 keys per round: lane (key t, quarter c) dots its quarter of the
 //     key codes with every head in fp32 and the quad adds the quarters.  The
 //     zero point's term sum_d q'_d k_zero_d is the same for every key of a head,
@@ -24,6 +25,12 @@
 //     Several chunks: (m, l, acc) partials go to the workspace with agent-scope
 //     stores and the last chunk of kv to arrive (agent-scope counter) merges
 //     them and resets the counter to zero.
+// Per token (TOK) a key's rulers are read by the lane that takes it in the softmax
+// (a wave has at most 64 keys): score = step (q . n) + min sum(q), weight p * V step,
+// and sum(p * V min) joins both dims of every lane.  All in fp32; the general
+// kernel, which served these calls and head_dim 80 before, holds its weights in 16
+// bits and walks 16-token tiles through two barriers each: 3000 tokens, 32 q / 8 KV
+// heads, 128 dims 47.4 -> 11.5 us per call (the host's part is 10).
 // use_quant = 0 attends over the raw codes.  Keys are loaded once, coalesced
 // (4 lanes per key row); V rows are staged in LDS for the byte-wise PV.
 #include "attention_kernel.h"
@@ -37,7 +44,8 @@ struct Params {
   const uint16_t* q;                        // [H, 1, D] fp16
   const uint8_t* kp;                        // [KV_t, S, D/2]
   const uint8_t* vp;
-  const uint16_t *ks, *vs, *vz;             // [KV_t, D] fp16
+  const uint16_t *ks, *vs, *vz;             // per channel: [KV_t, D] fp16
+  const uint16_t *tr[4];                    // per token: K min and step, V min and step, [KV_t, S] fp16
   float* out;                               // [H, 1, D]
   float* part;                              // [KV][nchunks][GT][D + 2] partials
   int* counters;                            // [KV] arrival counters (left at zero)
@@ -59,11 +67,12 @@ __device__ __forceinline__ float wave_sum(float x) {
   return a + b;
 }
 
-template <int D, int GT>
+template <int D, int GT, bool TOK>
 __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
-  constexpr int QB = D / 8;                 // key bytes per quarter lane
+  constexpr int QW = D / 64;                // 8-byte code words of a quarter lane: dims 16 QW c + 16 i ..
+  constexpr bool X = D == 80;               // and 2 bytes more, dims 64 + 4 c ..
   constexpr int VB = D / 2;                 // V bytes per key
-  constexpr int NB = D == 128 ? 64 : 32;    // lanes holding a head's output (dims 2b, 2b+1)
+  constexpr int NB = D == 64 ? 32 : 64;     // lanes of a key's V bytes (lane b: dims 2b, 2b+1; past VB: none)
   constexpr int HPW = (GT + NW - 1) / NW;   // heads each wave combines and writes
   __shared__ __attribute__((aligned(16))) float qs[GT * D];     // q' of the GT heads (zero past G)
   __shared__ __attribute__((aligned(16))) float sp[MAX_CT * 8];  // scores, then weights: [key][head]
@@ -71,6 +80,7 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
   __shared__ float wml[NW][GT][2];                                // each wave's (m, l) per head
   __shared__ __attribute__((aligned(16))) float2 wacc[NW][GT][64]; // each wave's PV sums per lane
   __shared__ float sw[HPW * NW][64];                              // merge coefficients per chunk
+  __shared__ float qsum[GT];                                      // per token: sum of the head's query
   __shared__ int last;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -89,18 +99,23 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
   // rows never read): selecting zeros instead made each load wait before the
   // next was issued.
   const int t = lane >> 2, c = lane & 3;
-  const uint8_t* kbase = p.kp + ((int64_t)kv * p.S + tok0 + wk0) * VB + c * QB;
-  const uint8_t* vbase = p.vp + ((int64_t)kv * p.S + tok0 + wk0) * VB + c * QB;
+  const uint8_t* kbase = p.kp + ((int64_t)kv * p.S + tok0 + wk0) * VB + c * 8 * QW;
+  const uint8_t* vbase = p.vp + ((int64_t)kv * p.S + tok0 + wk0) * VB + c * 8 * QW;
   struct Codes {
-    uint2 k[QB / 8], v[QB / 8];
+    uint2 k[QW], v[QW];
+    uint32_t kx, vx;
   };
   auto load_round = [&](int r) -> Codes {
     Codes cd;
     const int j = min(wk0 + 16 * r + t, ntok - 1) - wk0;   // a key of the chunk
 #pragma unroll
-    for (int i = 0; i < QB / 8; ++i) {
+    for (int i = 0; i < QW; ++i) {
       cd.k[i] = *reinterpret_cast<const uint2*>(kbase + (int64_t)j * VB + 8 * i);
       cd.v[i] = *reinterpret_cast<const uint2*>(vbase + (int64_t)j * VB + 8 * i);
+    }
+    if constexpr (X) {
+      cd.kx = *reinterpret_cast<const uint16_t*>(kbase + (int64_t)j * VB + 32 - 6 * c);
+      cd.vx = *reinterpret_cast<const uint16_t*>(vbase + (int64_t)j * VB + 32 - 6 * c);
     }
     return cd;
   };
@@ -110,23 +125,31 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
   // issued first, unconditionally (rows past G re-read the last head's, the
   // rulers are read without use_quant): under per-element branches each load
   // waited for the one before it.
-  const int b = lane % NB, par = lane / NB, step = 64 / NB;
+  const int b = min(lane % NB, VB - 1), par = lane / NB, step = 64 / NB;
+  const bool writes = lane < min(NB, VB);
   constexpr int QN = (GT * D + 64 * NW - 1) / (64 * NW);   // q' elements per thread
-  uint16_t qraw[QN], kraw[QN], vsr[2], vzw[2];
+  uint16_t qraw[QN], kraw[QN], vsr[2], vzw[2], tr[4];
 #pragma unroll
   for (int u = 0; u < QN; ++u) {
     const int i = min(tid + u * 64 * NW, GT * D - 1);
     const int h = min(i / D, p.G - 1), d = i % D;
     qraw[u] = p.q[(int64_t)(h0 + h) * D + d];
-    kraw[u] = p.ks[(int64_t)kv * D + d];
+    if constexpr (!TOK) kraw[u] = p.ks[(int64_t)kv * D + d];
   }
+  if constexpr (TOK) {
+    // rulers of the wave's key `lane` (a wave has at most 64), for the softmax
+    const int64_t at = (int64_t)kv * p.S + tok0 + min(wk0 + lane, ntok - 1);
 #pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    vsr[e] = p.vs[(int64_t)kv * D + 2 * b + e];
-    vzw[e] = p.vz[(int64_t)kv * D + 2 * b + e];
+    for (int i = 0; i < 4; ++i) tr[i] = p.tr[i][at];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      vsr[e] = p.vs[(int64_t)kv * D + 2 * b + e];
+      vzw[e] = p.vz[(int64_t)kv * D + 2 * b + e];
+    }
   }
   float vsc[2] = {1.f, 1.f}, vzr[2] = {0.f, 0.f};
-  if (quant) {
+  if (!TOK && quant) {
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       vsc[e] = h2f(vsr[e]);
@@ -137,29 +160,53 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
   for (int u = 0; u < QN; ++u) {
     const int i = tid + u * 64 * NW;
     if (i < GT * D) {
-      const float x = h2f(qraw[u]) * (quant ? h2f(kraw[u]) : 1.f);
+      float x = h2f(qraw[u]);
+      if constexpr (!TOK) x *= quant ? h2f(kraw[u]) : 1.f;
       qs[i] = i / D < p.G ? x : 0.f;
     }
   }
   __syncthreads();
+  if constexpr (TOK) {                      // (read in the softmax, a barrier later)
+#pragma unroll
+    for (int k = 0; k < HPW; ++k) {
+      const int h = wave + NW * k;
+      if (h >= GT) continue;
+      float x = 0.f;
+      for (int d = lane; d < D; d += 64) x += qs[h * D + d];
+      x = wave_sum(x);
+      if (lane == 0) qsum[h] = x;
+    }
+  }
 
   // ---- QK, 16 keys per round; V rows staged on the way
   for (int r = 0; r * 16 < wn; ++r) {
     const int jw = 16 * r + t;              // key within the wave's keys
     const int j = wk0 + jw;                 // key within the chunk
     if (r > 0) cur = load_round(r);
-    uint32_t kw[QB / 4];
+    uint32_t kw[2 * QW];
 #pragma unroll
-    for (int i = 0; i < QB / 8; ++i) {
-      *reinterpret_cast<uint2*>(vt + j * VB + c * QB + 8 * i) = cur.v[i];
+    for (int i = 0; i < QW; ++i) {
+      *reinterpret_cast<uint2*>(vt + j * VB + c * 8 * QW + 8 * i) = cur.v[i];
       kw[2 * i] = cur.k[i].x;
       kw[2 * i + 1] = cur.k[i].y;
     }
     float dot[GT];
 #pragma unroll
     for (int h = 0; h < GT; ++h) dot[h] = 0.f;
+    if constexpr (X) {
+      *reinterpret_cast<uint16_t*>(vt + j * VB + 32 + 2 * c) = (uint16_t)cur.vx;
+      const uint32_t x = cur.kx;
 #pragma unroll
-    for (int w = 0; w < QB / 4; ++w) {
+      for (int h = 0; h < GT; ++h) {
+        const float4 qa = *reinterpret_cast<const float4*>(&qs[h * D + 64 + 4 * c]);
+        float s = qa.x * (float)(x & 15u);
+        s = __builtin_fmaf(qa.y, (float)((x >> 4) & 15u), s);
+        s = __builtin_fmaf(qa.z, (float)((x >> 8) & 15u), s);
+        dot[h] = __builtin_fmaf(qa.w, (float)(x >> 12), s);
+      }
+    }
+#pragma unroll
+    for (int w = 0; w < 2 * QW; ++w) {
       float n[8];
 #pragma unroll
       for (int bb = 0; bb < 4; ++bb) {
@@ -167,7 +214,7 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
         n[2 * bb] = (float)(byte & 15u);
         n[2 * bb + 1] = (float)(byte >> 4);
       }
-      const int d0 = c * (D / 4) + 8 * w;
+      const int d0 = c * 16 * QW + 8 * w;
 #pragma unroll
       for (int h = 0; h < GT; ++h) {
         const float4 qa = *reinterpret_cast<const float4*>(&qs[h * D + d0]);
@@ -196,9 +243,24 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
 
   // ---- softmax per head over the wave's keys (base 2)
   const float kscale = 1.4426950408889634f * __builtin_amdgcn_rsqf((float)D);
-  float mh[GT], lh[GT];
+  float mh[GT], lh[GT], vt0[GT];             // vt0: per token, sum p * V min
+  if constexpr (TOK) {
+    const float kmin = h2f(tr[0]), kstep = h2f(tr[1]), vmin = h2f(tr[2]), vstep = h2f(tr[3]);
+    const int j = wk0 + lane;
 #pragma unroll
-  for (int h = 0; h < GT; ++h) {
+    for (int h = 0; h < GT; ++h) {
+      const float x = lane < wn ? __builtin_fmaf(sp[j * 8 + h], kstep, kmin * qsum[h]) * kscale : -INFINITY;
+      const float mx = wave_max(x);
+      // (scores of -inf alone: weight 0, as the wave's m of -inf says)
+      const float e = lane < wn ? __builtin_amdgcn_exp2f(x - (mx == -INFINITY ? 0.f : mx)) : 0.f;
+      if (lane < wn) sp[j * 8 + h] = e * vstep;
+      mh[h] = mx;
+      lh[h] = wave_sum(e);
+      vt0[h] = wave_sum(lane < wn ? e * vmin : 0.f);
+    }
+  }
+#pragma unroll
+  for (int h = 0; !TOK && h < GT; ++h) {
     float mx = -INFINITY;
     for (int j = lane; j < wn; j += 64) mx = fmaxf(mx, sp[(wk0 + j) * 8 + h] * kscale);
     mx = wave_max(mx);
@@ -242,6 +304,14 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
     }
   }
 
+  if constexpr (TOK) {
+#pragma unroll
+    for (int h = 0; h < GT; ++h) {
+      acc[h][0] += vt0[h];
+      acc[h][1] += vt0[h];
+    }
+  }
+
   // ---- the chunk's four waves combined (log-sum-exp) in LDS; wave w then
   // owns heads w, w + NW, ...
 #pragma unroll
@@ -280,7 +350,7 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
 
   auto write_out = [&](int h, float o0, float o1) {   // o: sum p * code / l, dims 2b, 2b+1
     const int d = 2 * b;
-    if (quant) {
+    if (!TOK && quant) {
       o0 = (o0 - vzr[0]) * vsc[0];
       o1 = (o1 - vzr[1]) * vsc[1];
     }
@@ -288,7 +358,7 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
   };
 
   if (p.nchunks == 1) {
-    if (lane < NB) {
+    if (writes) {
 #pragma unroll
       for (int k = 0; k < HPW; ++k) {
         const int h = wave + NW * k;
@@ -304,7 +374,7 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
   for (int k = 0; k < HPW; ++k) {
     const int h = wave + NW * k;
     if (h < GT) {
-      if (lane < NB) store_pair_agent(mypart + h * (D + 2) + 2 * b, ca[k].x, ca[k].y);
+      if (writes) store_pair_agent(mypart + h * (D + 2) + 2 * b, ca[k].x, ca[k].y);
       if (lane == 0) store_pair_agent(mypart + h * (D + 2) + D, cm[k], cl[k]);
     }
   }
@@ -365,24 +435,23 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
       swap32(o1, a0, a1);
       o1 = a0 + a1;
     }
-    if (lane < NB) write_out(h, o0, o1);
+    if (writes) write_out(h, o0, o1);
   }
   if (tid == 0) __hip_atomic_store(p.counters + kv, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int D, int GT>
+template <int D, int GT, bool TOK>
 int launch(const Params& p, int KV, hipStream_t stream) {
-  hipLaunchKernelGGL((split_kernel<D, GT>), dim3(p.nchunks, KV), dim3(64 * NW), 0, stream, p);
-  return check_launch("per-channel decode");
+  hipLaunchKernelGGL((split_kernel<D, GT, TOK>), dim3(p.nchunks, KV), dim3(64 * NW), 0, stream, p);
+  return check_launch(TOK ? "per-token decode" : "per-channel decode");
 }
 
 }  // namespace chan
 
-int launch_decode_channel_split(const void* q, const void* kp, const void* ks, const void* kz, const void* vp,
-                                const void* vs, const void* vz, int H, int G, int S, int D, int use_quant, float* out,
-                                void* workspace, int64_t ws_bytes, hipStream_t stream) {
-  (void)kz;   // the key zero point cancels in the softmax
-  if ((D != 64 && D != 128) || G < 1 || G > 8 || S < 1) return SLMT_ERR_UNSUPPORTED;
+int launch_decode_split(bool per_token, const void* q, const void* kp, const void* vp, const void* const* rulers, int H,
+                        int G, int S, int D, int use_quant, float* out, void* workspace, int64_t ws_bytes,
+                        hipStream_t stream) {
+  if (G < 1 || G > 8 || S < 1) return SLMT_ERR_UNSUPPORTED;
   const int KV = H / G;
   // chunk size: workgroups of four waves, each wave a multiple of 16 keys; the
   // smallest power of two from 64 keys per workgroup that gives at most 32
@@ -401,13 +470,19 @@ int launch_decode_channel_split(const void* q, const void* kp, const void* ks, c
   const int64_t part_off = kWsCounterInts * 4;
   if (nchunks > 1 && (workspace == nullptr || ws_bytes < part_off + part_bytes || KV > kWsCounterInts))
     return SLMT_ERR_UNSUPPORTED;
-  chan::Params p;
+  chan::Params p{};
   p.q = reinterpret_cast<const uint16_t*>(q);
   p.kp = reinterpret_cast<const uint8_t*>(kp);
   p.vp = reinterpret_cast<const uint8_t*>(vp);
-  p.ks = reinterpret_cast<const uint16_t*>(ks);
-  p.vs = reinterpret_cast<const uint16_t*>(vs);
-  p.vz = reinterpret_cast<const uint16_t*>(vz);
+  const uint16_t* r[4];
+  for (int i = 0; i < 4; ++i) r[i] = reinterpret_cast<const uint16_t*>(rulers[i]);
+  if (per_token) {
+    for (int i = 0; i < 4; ++i) p.tr[i] = r[i];
+  } else {   // the key zero point cancels in the softmax
+    p.ks = r[0];
+    p.vs = r[2];
+    p.vz = r[3];
+  }
   p.out = out;
   p.counters = reinterpret_cast<int*>(workspace);
   p.part = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(workspace) + part_off);
@@ -417,9 +492,10 @@ int launch_decode_channel_split(const void* q, const void* kp, const void* ks, c
   p.nchunks = nchunks;
   p.use_quant = use_quant ? 1 : 0;
 #define SLMT_CHAN_CASE(d, gt) \
-  if (D == d && GT == gt) return chan::launch<d, gt>(p, KV, stream);
-  SLMT_CHAN_CASE(64, 1) SLMT_CHAN_CASE(64, 2) SLMT_CHAN_CASE(64, 4) SLMT_CHAN_CASE(64, 8)
-  SLMT_CHAN_CASE(128, 1) SLMT_CHAN_CASE(128, 2) SLMT_CHAN_CASE(128, 4) SLMT_CHAN_CASE(128, 8)
+  if (D == d && GT == gt) return per_token ? chan::launch<d, gt, true>(p, KV, stream) : chan::launch<d, gt, false>(p, KV, stream);
+#define SLMT_CHAN_DIM(d) SLMT_CHAN_CASE(d, 1) SLMT_CHAN_CASE(d, 2) SLMT_CHAN_CASE(d, 4) SLMT_CHAN_CASE(d, 8)
+  SLMT_CHAN_DIM(64) SLMT_CHAN_DIM(80) SLMT_CHAN_DIM(128)
+#undef SLMT_CHAN_DIM
 #undef SLMT_CHAN_CASE
   return SLMT_ERR_UNSUPPORTED;
 }

@@ -272,14 +272,14 @@ int64_t attention_workspace_bytes(int B, int H, int KV, int D);
 // counters with partial results (each call leaves its counters at zero).
 constexpr int64_t kWsCounterInts = int64_t(1) << 20;
 
-// Single-sequence per-channel decode split over (KV head, key chunk)
-// workgroups (decode_channel.hip), head_dim 64 and 128, up to 8 query heads per
-// KV head and 16384 keys.  Returns SLMT_ERR_UNSUPPORTED (without an error
-// message) when the request falls outside that, so the caller can take the
-// general path.
-int launch_decode_channel_split(const void* q, const void* kp, const void* ks, const void* kz, const void* vp,
-                                const void* vs, const void* vz, int H, int G, int S, int D, int use_quant, float* out,
-                                void* workspace, int64_t ws_bytes, hipStream_t stream);
+// Single-sequence decode over contiguous per-channel or per-token buffers, split
+// over (KV head, key chunk) workgroups (decode_channel.hip), up to 8 query heads per
+// KV head and 16384 keys.  rulers: the entry point's four, in its order.  Returns
+// SLMT_ERR_UNSUPPORTED (without an error message) when the request falls outside
+// that, so the caller can take the general path.
+int launch_decode_split(bool per_token, const void* q, const void* kp, const void* vp, const void* const* rulers, int H,
+                        int G, int S, int D, int use_quant, float* out, void* workspace, int64_t ws_bytes,
+                        hipStream_t stream);
 
 // Per-channel prefill on the matrix cores (prefill_mfma.hip); no workspace.  q [H, M, D] fp16, codes [KV_t, S, D/2], rulers [KV_t, D].
 int launch_prefill_mfma(const void* q, const void* kp, const void* ks, const void* kz, const void* vp, const void* vs,

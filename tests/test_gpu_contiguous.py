@@ -391,3 +391,33 @@ def test_quantize_kv_row_counts(KV, S, D):
             _same_fp16(a.cpu().numpy(), b)
     for a, b in zip(alone, got):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+# Chunks of 64, 128 and 256 keys with remainders, one chunk, waves without keys, every
+# head-slot count, and head_dim 80 of both layouts; 20000 keys take the general path.
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,KV,D,S", [(1, 1, 64, 1), (8, 8, 128, 64), (8, 8, 80, 65), (14, 2, 64, 1025), (8, 4, 80, 2049),
+                                      (24, 6, 128, 3000), (32, 8, 80, 8000), (4, 2, 128, 16384), (4, 2, 64, 20000)])
+def test_decode_split_per_token_and_head_dim_80(H, KV, D, S):
+    """Weights and sums are fp32: 1e-5 of the output's size, against 64 bits."""
+    kd = _kd()
+    g = torch.Generator().manual_seed(S + D)
+    q = torch.randn(H, 1, D, generator=g).half()
+    kv = torch.randn(2, KV, S, D, generator=g).half()
+    packed = torch.randint(0, 256, (2, KV, S, D // 2), generator=g, dtype=torch.uint8)
+    mins, steps = kv.amin(-1), (torch.rand(2, KV, S, generator=g) * 0.4 + 0.05).half()
+    ref = oa.decode_per_token(q.numpy(), packed[0].numpy(), mins[0].numpy(), steps[0].numpy(), packed[1].numpy(),
+                                mins[1].numpy(), steps[1].numpy())
+    dev = "cuda:0"
+    t = [x.to(dev) for x in (packed[0], mins[0], steps[0], packed[1], mins[1], steps[1])]
+    atol = (1e-5 if S <= 16384 else 1e-3) * np.abs(ref).max()
+    for _ in range(2):
+        out = kd.kv_dequant_decode_per_token_attention(q.to(dev), *t)
+        assert_close(out.cpu().numpy(), ref, atol=atol, rtol=0, what="per-token split")
+    if D == 80:
+        scale, zero = (torch.rand(2, KV, D, generator=g) * 0.4 + 0.05).half(), torch.randint(0, 16, (2, KV, D), generator=g).half()
+        ref = oa.decode_per_channel(q.numpy(), packed[0].numpy(), scale[0].numpy(), zero[0].numpy(), packed[1].numpy(),
+                                      scale[1].numpy(), zero[1].numpy())
+        c = [x.to(dev) for x in (packed[0], scale[0], zero[0], packed[1], scale[1], zero[1])]
+        out = kd.kv_dequant_decode_attention(q.to(dev), *c)
+        assert_close(out.cpu().numpy(), ref, atol=1e-5 * np.abs(ref).max(), rtol=0, what="per-channel split, head_dim 80")
