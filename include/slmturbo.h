@@ -139,6 +139,32 @@ int slmt_decode_paged_batched(const void* q, int64_t q_seq_stride, int64_t q_hea
                               slmt_stream_t stream);
 
 /*
+ * Attention of a serving step's query tokens over the packed paged cache, some
+ * requests with more than one (a prefill chunk that continues cached context, several
+ * first chunks, decode tokens beside them); the reference leaves this unsupported
+ * (adapters/vllm_adapter.py:238-239).  Token t of request r (query_start_loc[r] <= t <
+ * query_start_loc[r + 1]) sits at position p = seq_lens[r] - query_len[r] + t -
+ * query_start_loc[r] and sees the keys 0 .. p of block-table row r, all of them in the
+ * cache already.
+ *   q, out:          as in slmt_decode_paged_batched, one row per token
+ *   kv_cache:        uint8 [num_blocks, block_size, KV, D+8]; block_size a power of
+ *                    two of at least 16
+ *   query_start_loc: int32 [num_reqs + 1], seq_lens: int32 [num_reqs], on the device;
+ *                    tokens past query_start_loc[num_reqs] are left alone
+ *   max_seq_len:     the longest of seq_lens or more; decides the split of the work only
+ * Tokens that see no key produce zeros.
+ * workspace: slmt_chunk_workspace_bytes of the same sizes; may be NULL where that is 0.
+ */
+int64_t slmt_chunk_workspace_bytes(int64_t num_tokens, int num_reqs, int num_heads, int num_kv_heads, int head_dim,
+                                   int max_seq_len);
+int slmt_chunk_paged(const void* q, int64_t q_token_stride, int64_t q_head_stride, const void* kv_cache,
+                     int64_t num_blocks, int block_size, const void* block_tables, int block_table_bits,
+                     int64_t block_table_stride, const int32_t* query_start_loc, const int32_t* seq_lens,
+                     int max_seq_len, int num_tokens, int num_reqs, int num_heads, int num_kv_heads, int head_dim,
+                     void* out, int out_dtype, int64_t out_token_stride, int64_t out_head_stride, void* workspace,
+                     int64_t workspace_bytes, slmt_stream_t stream);
+
+/*
  * Allocation-free batched paged decode.  No counterpart in the reference: it
  * is for callers that cannot allocate device memory or pass a workspace (code
  * under HIP graph capture, tight serving loops, harnesses that forbid

@@ -66,6 +66,10 @@ def packed_kv_cache_shape(num_blocks: int, block_size: int, num_kv_heads: int, h
     return (num_blocks, block_size, num_kv_heads, head_size + 8)
 
 
+def _int32(t):
+    return t if t.dtype is torch.int32 else t.to(torch.int32)
+
+
 def packed_slot_bytes(head_size: int) -> int:
     return head_size + 8
 
@@ -172,9 +176,29 @@ class PackedKVAttentionMixin:
         adapters/vllm_adapter.py:238-239).  Query
         token i of request r sits at absolute position p = seq_len[r] -
         query_len[r] + (i - query_start[r]) and attends to tokens [0, p] of r,
-        all of which this step's do_kv_cache_update has already written.  Each
-        query token becomes one sequence of length p + 1 with r's block-table
-        row: one batched launch, index arithmetic on the device, no host sync."""
+        all of which this step's do_kv_cache_update has already written.  No host sync.
+
+        The chunk kernel reads a request's keys once per 64 (token, query head) rows of
+        a KV head; the batched decode, each query token a sequence of length p + 1 with
+        r's block-table row, once per token.  The first costs as much per request as two
+        to five sequences of the second where it has few rows, so it takes steps of
+        five tokens per request and more (one and a half at head_dim 64), and short ones,
+        for which the other's index arithmetic takes longer.  us, 2 / 4 / 6 tokens each
+        (first against second), 32 q / 8 KV heads, 128 dims: 32 requests of 3000 tokens
+        72 / 75 against 82 / 105, 64 of 8000 254 / 243 / 280 against 209 / 377 / 548; 32
+        / 4 heads, 64 dims, 64 of 8000 90 / 103 / 191 against 118 / 201 / 286."""
+        block_size, num_kv_heads = kv_cache.shape[1], kv_cache.shape[2]
+        R = attn_metadata.query_start_loc.numel() - 1
+        most = int(attn_metadata.max_seq_len)
+        if (query.is_cuda and 16 <= block_size <= 1024 and block_size & (block_size - 1) == 0
+                and (N * most <= 200_000 or 2 * N >= (3 if self.head_size == 64 else 10) * R)):
+            kd = self._slm_kernels()
+            seq_lens, tables = attn_metadata.seq_lens[:R], attn_metadata.block_table[:R]
+            qsl = attn_metadata.query_start_loc
+            self._into_output(output, N, lambda out, dtype: kd.kv_dequant_chunk_paged(
+                query, kv_cache, tables, _int32(seq_lens), _int32(qsl), most, block_size, num_kv_heads, out=out,
+                out_dtype=dtype))
+            return
         qsl = attn_metadata.query_start_loc.to(torch.int64)       # [R+1]
         R = qsl.numel() - 1
         tok = torch.arange(N, device=query.device, dtype=torch.int64)
@@ -195,22 +219,21 @@ class PackedKVAttentionMixin:
 
     def _paged_attention(self, query, kv_cache, seq_lens, block_table, output, N):
         """One batched paged decode launch: query row n attends to the first
-        seq_lens[n] tokens of block-table row n.  Writes output[:N] (in place
-        when the output buffer allows)."""
-        global _KERNEL_CALLS, _KERNEL_LAUNCHES
+        seq_lens[n] tokens of block-table row n.  Writes output[:N]."""
         kd = self._slm_kernels()
         block_size, num_kv_heads = kv_cache.shape[1], kv_cache.shape[2]
-        if seq_lens.dtype != torch.int32:
-            seq_lens = seq_lens.to(torch.int32)
+        self._into_output(output, N, lambda out, dtype: kd.kv_dequant_decode_paged_batched(
+            query, kv_cache, block_table, _int32(seq_lens), block_size, num_kv_heads, out=out, out_dtype=dtype))
+
+    def _into_output(self, output, N, attend):
+        """output[:N] from attend(out, out_dtype): in place when the output buffer
+        allows, else from an fp32 result."""
+        global _KERNEL_CALLS, _KERNEL_LAUNCHES
         H, D = self.num_heads, self.head_size
-        out3 = None
         if output.dtype in (torch.float16, torch.float32) and output.is_contiguous():
-            out3 = output[:N].view(N, H, D)        # written in place
-        res = kd.kv_dequant_decode_paged_batched(query, kv_cache, block_table, seq_lens, block_size,
-                                                 num_kv_heads, out=out3,
-                                                 out_dtype=None if out3 is not None else torch.float32)
-        if out3 is None:
-            self._store_output(output, res, N)
+            attend(output[:N].view(N, H, D), None)
+        else:
+            self._store_output(output, attend(None, torch.float32), N)
         _KERNEL_CALLS += N
         _KERNEL_LAUNCHES += 1
         if not getattr(self, "_slm_logged", False):       # once per layer implementation, as the reference

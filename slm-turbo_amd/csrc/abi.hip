@@ -245,6 +245,65 @@ int slmt_decode_paged_batched(const void* q, int64_t q_seq_stride, int64_t q_hea
                               workspace_bytes, reinterpret_cast<hipStream_t>(stream), false);
 }
 
+int64_t slmt_chunk_workspace_bytes(int64_t num_tokens, int num_reqs, int num_heads, int num_kv_heads, int head_dim,
+                                   int max_seq_len) {
+  clear_error();
+  if (!head_dim_ok(head_dim)) return fail(SLMT_ERR_INVALID, "workspace: head_dim must be 64/80/128, got " + s(head_dim)), -1;
+  if (num_tokens < 0 || num_reqs < 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0)
+    return fail(SLMT_ERR_INVALID, "workspace: invalid sizes"), -1;
+  return chunk_workspace_bytes(num_tokens, num_reqs, num_heads, num_kv_heads, head_dim, max_seq_len);
+}
+
+int slmt_chunk_paged(const void* q, int64_t q_token_stride, int64_t q_head_stride, const void* kv_cache,
+                     int64_t num_blocks, int block_size, const void* block_tables, int block_table_bits,
+                     int64_t block_table_stride, const int32_t* query_start_loc, const int32_t* seq_lens,
+                     int max_seq_len, int num_tokens, int num_reqs, int num_heads, int num_kv_heads, int head_dim,
+                     void* out, int out_dtype, int64_t out_token_stride, int64_t out_head_stride, void* workspace,
+                     int64_t workspace_bytes, slmt_stream_t stream) {
+  clear_error();
+  if (!head_dim_ok(head_dim)) return fail(SLMT_ERR_INVALID, "chunk: head_dim must be 64/80/128, got " + s(head_dim));
+  if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0)
+    return fail(SLMT_ERR_INVALID, "H not divisible by num_kv_heads");
+  const int shift = block_shift_of(block_size);
+  if (shift < 4) return fail(SLMT_ERR_INVALID, "chunk: block_size must be a power of two of at least 16, got " + s(block_size));
+  if (block_table_bits != 32 && block_table_bits != 64)
+    return fail(SLMT_ERR_INVALID, "chunk: block table must be int32 or int64");
+  if (out_dtype != SLMT_OUT_F32 && out_dtype != SLMT_OUT_F16)
+    return fail(SLMT_ERR_INVALID, "chunk: out dtype must be fp32 or fp16");
+  if (num_tokens < 0 || num_reqs < 0 || num_blocks < 0 || num_blocks >= (int64_t(1) << 31))
+    return fail(SLMT_ERR_INVALID, "chunk: invalid sizes");
+  if ((int64_t)num_tokens * (num_heads / num_kv_heads) >= (int64_t(1) << 31) - 64)
+    return fail(SLMT_ERR_UNSUPPORTED, "chunk: too many query rows for one launch");
+  if (num_tokens == 0 || num_reqs == 0) return SLMT_OK;
+  if (!q || !kv_cache || !block_tables || !query_start_loc || !seq_lens || !out)
+    return fail(SLMT_ERR_INVALID, "chunk: null pointer argument");
+  if (!aligned(q, 16) || (q_token_stride % 8) || (q_head_stride % 8))
+    return fail(SLMT_ERR_INVALID, "chunk: q must be 16-byte aligned with strides that are multiples of 8");
+  if (!aligned(out, out_dtype == SLMT_OUT_F32 ? 8 : 4) || (out_token_stride & 1) || (out_head_stride & 1))
+    return fail(SLMT_ERR_INVALID, "chunk: out must be aligned with even strides");
+  if (!aligned(kv_cache, 8)) return fail(SLMT_ERR_INVALID, "chunk: kv_cache must be 8-byte aligned");
+  ChunkParams p{};
+  p.q = reinterpret_cast<const uint16_t*>(q);
+  p.q_seq_stride = q_token_stride;
+  p.q_head_stride = q_head_stride;
+  p.cache = reinterpret_cast<const uint8_t*>(kv_cache);
+  p.block_tables = block_tables;
+  p.bt_stride = block_table_stride;
+  p.bt64 = block_table_bits == 64;
+  p.block_shift = shift;
+  p.query_start = query_start_loc;
+  p.seq_lens = seq_lens;
+  p.N = num_tokens;
+  p.R = num_reqs;
+  p.G = num_heads / num_kv_heads;
+  p.KV = num_kv_heads;
+  p.out = out;
+  p.out_f16 = out_dtype == SLMT_OUT_F16;
+  p.out_seq_stride = out_token_stride;
+  p.out_head_stride = out_head_stride;
+  return launch_chunk(head_dim, p, max_seq_len, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
+}
+
 int slmt_decode_paged(const void* q, const void* kv_cache, int64_t num_blocks, int block_size,
                       const int64_t* block_table, int seq_len, int num_heads, int num_kv_heads,
                       int head_dim, float* out, void* workspace, int64_t workspace_bytes,
@@ -274,6 +333,10 @@ int slmt_decode_per_token(const void* q, const void* k_packed, const void* k_min
   if (rc != SLMT_OK) return rc;
   rc = check_workspace(ph, 1, num_heads, num_kv_heads, head_dim, workspace, workspace_bytes);
   if (rc != SLMT_OK) return rc;
+  // one short sequence: split over (KV head, key chunk) when the shape allows it
+  rc = launch_decode_split(true, q, k_packed, v_packed, r, num_heads, num_heads / num_kv_heads, seq_len, head_dim, 1,
+                           out, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
+  if (rc != SLMT_ERR_UNSUPPORTED) return rc;
   AttnParams p = blank_params();
   p.q = reinterpret_cast<const uint16_t*>(q);
   p.q_seq_stride = (int64_t)num_heads * head_dim;
@@ -332,10 +395,6 @@ int slmt_decode_per_channel(const void* q, const void* k_packed, const void* k_s
   p.out = out;
   p.out_seq_stride = (int64_t)num_heads * head_dim;
   p.out_head_stride = head_dim;
-  // one short sequence: split over (KV head, key chunk) when the shape allows it
-  rc = launch_decode_split(true, q, k_packed, v_packed, r, num_heads, num_heads / num_kv_heads, seq_len, head_dim, 1,
-                           out, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
-  if (rc != SLMT_ERR_UNSUPPORTED) return rc;
   return launch_attention(SRC_CHANNEL, head_dim, p, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
 }
 

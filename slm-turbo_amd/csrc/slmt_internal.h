@@ -281,6 +281,27 @@ int launch_decode_split(bool per_token, const void* q, const void* kp, const voi
                         int G, int S, int D, int use_quant, float* out, void* workspace, int64_t ws_bytes,
                         hipStream_t stream);
 
+// Chunked prefill over the packed paged cache (chunk_mfma.hip).
+struct ChunkParams {
+  const uint16_t* q;               // element (token, h, d) at q + token*q_seq_stride + h*q_head_stride + d
+  int64_t q_seq_stride, q_head_stride;
+  const uint8_t* cache;
+  const void* block_tables;
+  int64_t bt_stride;
+  int bt64, block_shift;
+  const int32_t *query_start, *seq_lens;   // [R + 1], [R]
+  int N, R, G, KV;
+  void* out;
+  int out_f16;
+  int64_t out_seq_stride, out_head_stride;
+  // the split of long contexts: parts of split_tiles 64-key tiles, and their partials
+  int nsplit, split_tiles;
+  float* part_o;                   // [block][KV][part][64 columns][D]
+  float* part_ml;                  // [block][KV][part][64 columns][2]
+};
+int64_t chunk_workspace_bytes(int64_t N, int R, int H, int KV, int D, int max_seq_len);
+int launch_chunk(int D, ChunkParams& p, int max_seq_len, void* workspace, int64_t ws_bytes, hipStream_t stream);
+
 // Per-channel prefill on the matrix cores (prefill_mfma.hip); no workspace.  q [H, M, D] fp16, codes [KV_t, S, D/2], rulers [KV_t, D].
 int launch_prefill_mfma(const void* q, const void* kp, const void* ks, const void* kz, const void* vp, const void* vs,
                         const void* vz, int H, int G, int M, int S, int D, int causal, int use_quant, float* out,

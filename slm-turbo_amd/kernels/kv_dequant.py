@@ -39,6 +39,7 @@ __all__ = [
     "kv_quantize_store",
     "kv_dequant_decode_per_token_paged_attention",
     "kv_dequant_decode_paged_batched",
+    "kv_dequant_chunk_paged",
     "quantize_per_channel",
     "quantize_kv",
 ]
@@ -98,7 +99,12 @@ def _workspace(lib, device: torch.device, B: int, H: int, KV: int, D: int,
         if need < 0:
             raise RuntimeError(_native.last_error(lib))
         _need_cache[nkey] = need
-    key = (device.index, _stream(device) if stream is None else stream)
+    return _workspace_of(device, need, _stream(device) if stream is None else stream)
+
+
+def _workspace_of(device: torch.device, need: int, stream: int) -> tuple[int, int]:
+    """The stream's scratch buffer, of ``need`` bytes or more."""
+    key = (device.index, stream)
     buf = _ws_cache.get(key)
     if buf is None or buf.numel() < need:
         with _ws_lock:
@@ -449,6 +455,84 @@ def kv_dequant_decode_paged_batched(
             seq_lens.data_ptr(), 0, B, H, num_kv_heads, D, out.data_ptr(),
             _native.OUT_F16 if out_dtype is torch.float16 else _native.OUT_F32,
             out_stride[0], out_stride[1], ws, ws_bytes, stream)
+        if rc:
+            _native.check(lib, rc)
+    return out
+
+
+# =============================================================================
+#  CHUNKED PREFILL over the packed paged cache (a serving step's query tokens)
+# =============================================================================
+def kv_dequant_chunk_paged(
+    q, kv_cache, block_tables, seq_lens, query_start_loc, max_seq_len, block_size, num_kv_heads, out=None,
+    out_dtype=None,
+):
+    """Attention of a step's query tokens over the packed cache.  Returns [N, H, D].
+
+    Token t of request r sees the first seq_lens[r] - query_len[r] + (t -
+    query_start_loc[r]) + 1 tokens of block-table row r (no counterpart in the
+    reference, adapters/vllm_adapter.py:238-239):
+        q               [N, H, D] fp16 (strides: any, with unit stride over D)
+        kv_cache        [num_blocks, block_size, KV, D+8] uint8, block_size a power of
+                        two of at least 16
+        block_tables    [R, max_blocks] int32 or int64 (device)
+        seq_lens        [R] int32, query_start_loc [R + 1] int32 (device; read by
+                        the kernel, no host sync)
+        max_seq_len     the longest of seq_lens, or more
+        out, out_dtype  as in kv_dequant_decode_paged_batched
+    Tokens that see no key produce zeros.
+    """
+    assert q.dim() == 3, f"q must be [N, H, D], got {tuple(q.shape)}"
+    N, H, D = q.shape
+    assert D in (64, 80, 128), f"head_dim must be 64/80/128, got {D}"
+    assert H % num_kv_heads == 0, f"H {H} not divisible by num_kv_heads {num_kv_heads}"
+    cshape = kv_cache.shape
+    assert cshape[-1] == D + 8, f"cache slot must be D+8, got {cshape[-1]}"
+    lib = _load_native_extension()
+    if not (q.is_cuda and q.dtype is torch.float16):
+        raise RuntimeError("paged decode: q must be fp16 CUDA")
+    if not (kv_cache.is_cuda and kv_cache.dtype is torch.uint8 and kv_cache.is_contiguous()):
+        raise RuntimeError("paged decode: kv_cache must be a contiguous uint8 CUDA tensor")
+    if not (len(cshape) == 4 and cshape[1] == block_size and cshape[2] == num_kv_heads):
+        raise RuntimeError(f"paged decode: kv_cache must be [num_blocks, {block_size}, {num_kv_heads}, {D + 8}]")
+    R = query_start_loc.numel() - 1
+    bt_dtype = block_tables.dtype
+    if not (block_tables.dim() == 2 and block_tables.size(0) == R and block_tables.is_cuda
+            and (bt_dtype is torch.int32 or bt_dtype is torch.int64)):
+        raise RuntimeError("paged decode: block_tables must be an int32/int64 CUDA tensor [R, max_blocks]")
+    for t, n in ((seq_lens, R), (query_start_loc, R + 1)):
+        if not (t.is_cuda and t.dtype is torch.int32 and t.numel() == n):
+            raise RuntimeError("paged decode: seq_lens [R] and query_start_loc [R + 1] must be int32 CUDA tensors")
+    dev = q.device
+    with _on_device(dev):
+        if out is None:
+            out = torch.empty((N, H, D), dtype=out_dtype or torch.float32, device=dev)
+        out_dtype = out.dtype
+        out_stride = out.stride()
+        if not ((out_dtype is torch.float32 or out_dtype is torch.float16) and out.shape == (N, H, D)
+                and out_stride[2] == 1):
+            raise RuntimeError("paged decode: out must be fp32/fp16 [N, H, D] with unit stride over D")
+        if N == 0:
+            return out
+        qs = q.stride()
+        if qs[2] != 1 or qs[1] % 8 or qs[0] % 8 or q.data_ptr() % 16:
+            q = q.contiguous()
+            qs = q.stride()
+        if block_tables.stride(1) != 1:
+            block_tables = block_tables.contiguous()
+        seq_lens, query_start_loc = seq_lens.contiguous(), query_start_loc.contiguous()
+        stream = _stream(dev)
+        max_seq_len = min(max(int(max_seq_len), 1), 2**31 - 1)
+        need = lib.slmt_chunk_workspace_bytes(N, R, H, num_kv_heads, D, max_seq_len)
+        if need < 0:
+            raise RuntimeError(_native.last_error(lib))
+        ws, ws_bytes = _workspace_of(dev, need, stream) if need else (0, 0)
+        rc = lib.slmt_chunk_paged(
+            q.data_ptr(), qs[0], qs[1], kv_cache.data_ptr(), cshape[0], int(block_size), block_tables.data_ptr(),
+            64 if bt_dtype is torch.int64 else 32, block_tables.stride(0), query_start_loc.data_ptr(),
+            seq_lens.data_ptr(), max_seq_len, N, R, H, num_kv_heads, D, out.data_ptr(),
+            _native.OUT_F16 if out_dtype is torch.float16 else _native.OUT_F32, out_stride[0], out_stride[1],
+            ws, ws_bytes, stream)
         if rc:
             _native.check(lib, rc)
     return out

@@ -336,3 +336,62 @@ def test_store_row_remainders_and_special_values(N, KV, D):
     kd.kv_quantize_store(k, v, cache, slots.to("cuda:0"), 16)
     torch.cuda.synchronize()
     assert np.array_equal(cache.cpu().numpy(), ref)
+
+
+# Query blocks of 64 rows with remainders (rows of one token on both sides of a block),
+# blocks of 16 to 128 tokens, first chunks, decode tokens, requests without tokens,
+# contexts that are split and that are not, and a context that ends on a tile.
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,KV,D,bs,lens,qlens", [
+    (14, 2, 64, 16, [40, 700, 64], [17, 64, 1]),
+    (8, 8, 80, 16, [129, 30, 1], [65, 30, 1]),
+    (32, 8, 80, 32, [900, 17, 300], [33, 2, 0]),
+    (12, 2, 128, 64, [2000, 5, 128], [11, 5, 128]),
+    (24, 3, 64, 16, [5000], [24]),
+    (5, 5, 128, 128, [200, 150], [130, 20]),
+    (64, 1, 64, 16, [70, 3], [3, 1]),
+])
+def test_chunk_matches_oracle(H, KV, D, bs, lens, qlens):
+    """fp32 results: codes and query are exact operands, weights carry ~22 bits, so
+    1e-5 of the output's size."""
+    kd = _kd()
+    case = make_paged_case(seed=sum(lens), B=len(lens), H=H, KV=KV, D=D, lens=lens, block_size=bs, dist="t3")
+    N = sum(qlens)
+    g = torch.Generator().manual_seed(N)
+    fused = torch.randn(N, H * D + 16, generator=g).half()
+    q = fused[:, 8:8 + H * D].unflatten(1, (H, D))
+    rows = torch.cat([case.block_tables[r][None].expand(n, -1) for r, n in enumerate(qlens)])
+    vlens = [L - n + i + 1 for L, n in zip(lens, qlens) for i in range(n)]
+    ref = paged_reference(type(case)(q=q, kv_cache=case.kv_cache, block_tables=rows,
+                                     seq_lens=torch.tensor(vlens, dtype=torch.int32), block_size=bs, num_kv_heads=KV))
+    dev = "cuda:0"
+    qsl = torch.tensor([0] + qlens).cumsum(0).to(torch.int32).to(dev)
+    cache, tables = torch.from_numpy(case.kv_cache).to(dev), case.block_tables.to(dev)
+    qd = fused.to(dev)[:, 8:8 + H * D].unflatten(1, (H, D))
+    for bt, f16 in ((tables, False), (tables.long(), True)):
+        out = kd.kv_dequant_chunk_paged(qd, cache, bt, case.seq_lens.to(dev), qsl, max(lens), bs, KV,
+                                        out_dtype=torch.float16 if f16 else torch.float32)
+        torch.cuda.synchronize()
+        atol = 1e-5 * np.abs(ref).max()
+        assert_close(out.float().cpu().numpy(), ref, atol=atol, rtol=5e-4 if f16 else 0, what="chunk")
+
+
+@pytest.mark.gpu
+def test_chunk_slots_past_a_position_stay_out():
+    """Rulers of tokens past a query's position (NaN here) reach no earlier query, and a
+    longest length that is too small loses no keys."""
+    kd = _kd()
+    case = make_paged_case(seed=5, B=1, H=8, KV=2, D=64, lens=[600], extra_blocks=1)
+    q = torch.randn(40, 8, 64, generator=torch.Generator().manual_seed(6)).half()
+    bad = case.kv_cache.copy()
+    for pos in range(580, 600):
+        bad[int(case.block_tables[0, pos // 16]), pos % 16, :, 64:] = 0x7F      # fp16 NaNs
+    ref = paged_reference(type(case)(q=q, kv_cache=case.kv_cache, block_tables=case.block_tables.expand(40, -1),
+                                     seq_lens=torch.arange(561, 601, dtype=torch.int32), block_size=16, num_kv_heads=2))
+    dev = "cuda:0"
+    for most in (600, 100):
+        out = kd.kv_dequant_chunk_paged(q.to(dev), torch.from_numpy(bad).to(dev), case.block_tables.to(dev),
+                                        case.seq_lens.to(dev), torch.tensor([0, 40], dtype=torch.int32, device=dev), most, 16, 2)
+        out = out.cpu().numpy()
+        assert_close(out[:20], ref[:20], atol=1e-5 * np.abs(ref).max(), rtol=0, what="before the NaNs")
+        assert np.isnan(out[20:]).all()
