@@ -70,6 +70,11 @@ def _int32(t):
     return t if t.dtype is torch.int32 else t.to(torch.int32)
 
 
+def _first(t, n):
+    """t[:n] (t itself where that is all of it: a slice costs the host a microsecond)."""
+    return t if t.shape[0] == n else t[:n]
+
+
 def packed_slot_bytes(head_size: int) -> int:
     return head_size + 8
 
@@ -118,7 +123,7 @@ class PackedKVAttentionMixin:
         N = int(attn_metadata.num_actual_tokens)
         if N <= 0:
             return output.fill_(0)
-        q = query[:N]
+        q = _first(query, N)
         if int(attn_metadata.max_query_len) > 1:
             if self._one_first_chunk(attn_metadata):
                 attn_out = self._prefill_attention(q, key[:N], value[:N], kv_cache, attn_metadata)
@@ -193,7 +198,7 @@ class PackedKVAttentionMixin:
         if (query.is_cuda and 16 <= block_size <= 1024 and block_size & (block_size - 1) == 0
                 and (N * most <= 200_000 or 2 * N >= (3 if self.head_size == 64 else 10) * R)):
             kd = self._slm_kernels()
-            seq_lens, tables = attn_metadata.seq_lens[:R], attn_metadata.block_table[:R]
+            seq_lens, tables = _first(attn_metadata.seq_lens, R), _first(attn_metadata.block_table, R)
             qsl = attn_metadata.query_start_loc
             self._into_output(output, N, lambda out, dtype: kd.kv_dequant_chunk_paged(
                 query, kv_cache, tables, _int32(seq_lens), _int32(qsl), most, block_size, num_kv_heads, out=out,
@@ -214,8 +219,8 @@ class PackedKVAttentionMixin:
         """query [N, H, D] (one token per request), kv_cache [nb, bs, KV, D+8]
         uint8; reads attn_metadata.seq_lens [N] and .block_table [N, max]
         on the device.  Writes output[:N]."""
-        self._paged_attention(query, kv_cache, attn_metadata.seq_lens[:N], attn_metadata.block_table[:N],
-                              output, N)
+        self._paged_attention(query, kv_cache, _first(attn_metadata.seq_lens, N),
+                              _first(attn_metadata.block_table, N), output, N)
 
     def _paged_attention(self, query, kv_cache, seq_lens, block_table, output, N):
         """One batched paged decode launch: query row n attends to the first
@@ -231,7 +236,7 @@ class PackedKVAttentionMixin:
         global _KERNEL_CALLS, _KERNEL_LAUNCHES
         H, D = self.num_heads, self.head_size
         if output.dtype in (torch.float16, torch.float32) and output.is_contiguous():
-            attend(output[:N].view(N, H, D), None)
+            attend(_first(output, N).view(N, H, D), None)
         else:
             self._store_output(output, attend(None, torch.float32), N)
         _KERNEL_CALLS += N

@@ -1,22 +1,15 @@
 /*
- * _slmt_fast: a CPython METH_FASTCALL binding of the two per-layer hot entry
- * points of libslmturbo_hip.so (slmt_quantize_store, slmt_decode_paged_batched).
- * ctypes spends ~3 us converting a dozen arguments per call; this module takes
- * the same arguments as plain Python ints (pointers as integers) and calls the
- * library through function pointers that kernels/_native.py hands it from the
- * loaded library (bind), so the two bindings always reach the same code.
+ * _slmt_fast: a CPython METH_FASTCALL binding of the hot entry points of
+ * libslmturbo_hip.so.  ctypes spends ~3 us converting a dozen arguments per call;
+ * this module takes the same arguments as plain Python ints (pointers as integers)
+ * and calls the library through function pointers that kernels/_native.py hands it
+ * from the loaded library (bind), so the two bindings always reach the same code.
  * Host code only: no device work happens here.
  */
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
 #include "../../include/slmturbo.h"
-
-typedef __typeof__(slmt_quantize_store) store_fn;
-typedef __typeof__(slmt_decode_paged_batched) decode_fn;
-
-static store_fn* g_store = NULL;
-static decode_fn* g_decode = NULL;
 
 /* args[i] as a 64-bit integer; -1 with an exception set on failure */
 static int take(PyObject* const* args, Py_ssize_t n, long long* v) {
@@ -27,66 +20,86 @@ static int take(PyObject* const* args, Py_ssize_t n, long long* v) {
   return 0;
 }
 
+#define P(i) ((void*)(intptr_t)v[i])
+#define I(i) ((int)v[i])
+#define L(i) ((int64_t)v[i])
+
+/* One function: N integer arguments, handed on as the entry point's own types. */
+#define ENTRY(name, N, ...)                                                        \
+  static __typeof__(slmt_##name)* g_##name = NULL;                                 \
+  static PyObject* name(PyObject* self, PyObject* const* args, Py_ssize_t n) {     \
+    (void)self;                                                                    \
+    long long v[N];                                                                \
+    if (!g_##name) {                                                               \
+      PyErr_SetString(PyExc_RuntimeError, #name ": library not bound");            \
+      return NULL;                                                                 \
+    }                                                                              \
+    if (n != N) {                                                                  \
+      PyErr_SetString(PyExc_TypeError, #name " takes " #N " arguments");           \
+      return NULL;                                                                 \
+    }                                                                              \
+    if (take(args, N, v)) return NULL;                                             \
+    return PyLong_FromLongLong(g_##name(__VA_ARGS__));                             \
+  }
+
+ENTRY(quantize_store, 12, P(0), L(1), P(2), L(3), P(4), L(5), I(6), P(7), L(8), I(9), I(10), P(11))
+ENTRY(decode_paged_batched, 22, P(0), L(1), L(2), P(3), L(4), I(5), P(6), I(7), L(8), P(9), I(10), I(11),
+      I(12), I(13), I(14), P(15), I(16), L(17), L(18), P(19), L(20), P(21))
+ENTRY(chunk_paged, 24, P(0), L(1), L(2), P(3), L(4), I(5), P(6), I(7), L(8), P(9), P(10), I(11), I(12), I(13),
+      I(14), I(15), I(16), P(17), I(18), L(19), L(20), P(21), L(22), P(23))
+ENTRY(chunk_workspace_bytes, 6, L(0), I(1), I(2), I(3), I(4), I(5))
+ENTRY(decode_per_token, 17, P(0), P(1), P(2), P(3), P(4), P(5), P(6), I(7), I(8), I(9), I(10), I(11), I(12),
+      P(13), P(14), L(15), P(16))
+ENTRY(decode_per_channel, 18, P(0), P(1), P(2), P(3), P(4), P(5), P(6), I(7), I(8), I(9), I(10), I(11), I(12),
+      I(13), P(14), P(15), L(16), P(17))
+ENTRY(prefill_per_channel, 21, P(0), P(1), P(2), P(3), P(4), P(5), P(6), I(7), I(8), I(9), I(10), I(11),
+      I(12), I(13), I(14), I(15), I(16), P(17), P(18), L(19), P(20))
+ENTRY(quantize_kv_per_channel, 12, P(0), P(1), I(2), I(3), I(4), P(5), P(6), P(7), P(8), P(9), P(10), P(11))
+ENTRY(quantize_with_rulers, 12, P(0), L(1), L(2), I(3), I(4), I(5), P(6), P(7), P(8), L(9), L(10), P(11))
+
+/* bind(name, address): the library's entry point slmt_<name> */
 static PyObject* bind(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   (void)self;
-  long long v[2];
-  if (n != 2) {
-    PyErr_SetString(PyExc_TypeError, "bind(store_address, decode_address)");
+  long long at;
+  if (n != 2 || !PyUnicode_Check(args[0])) {
+    PyErr_SetString(PyExc_TypeError, "bind(name, address)");
     return NULL;
   }
-  if (take(args, 2, v)) return NULL;
-  if (!v[0] || !v[1]) {
+  if (take(args + 1, 1, &at)) return NULL;
+  if (!at) {
     PyErr_SetString(PyExc_ValueError, "bind: null function address");
     return NULL;
   }
-  g_store = (store_fn*)(intptr_t)v[0];
-  g_decode = (decode_fn*)(intptr_t)v[1];
-  Py_RETURN_NONE;
+#define BIND(name)                                                  \
+  if (PyUnicode_CompareWithASCIIString(args[0], #name) == 0) {      \
+    g_##name = (__typeof__(slmt_##name)*)(intptr_t)at;              \
+    Py_RETURN_NONE;                                                 \
+  }
+  BIND(quantize_store)
+  BIND(decode_paged_batched)
+  BIND(chunk_paged)
+  BIND(chunk_workspace_bytes)
+  BIND(decode_per_token)
+  BIND(decode_per_channel)
+  BIND(prefill_per_channel)
+  BIND(quantize_kv_per_channel)
+  BIND(quantize_with_rulers)
+  PyErr_SetString(PyExc_ValueError, "bind: no such entry point");
+  return NULL;
 }
 
-static PyObject* quantize_store(PyObject* self, PyObject* const* args, Py_ssize_t n) {
-  (void)self;
-  long long v[12];
-  if (!g_store) {
-    PyErr_SetString(PyExc_RuntimeError, "quantize_store: library not bound");
-    return NULL;
-  }
-  if (n != 12) {
-    PyErr_SetString(PyExc_TypeError, "quantize_store takes 12 arguments");
-    return NULL;
-  }
-  if (take(args, 12, v)) return NULL;
-  const int rc = g_store((const void*)(intptr_t)v[0], (int64_t)v[1], (const void*)(intptr_t)v[2], (int64_t)v[3],
-                         (void*)(intptr_t)v[4], (int64_t)v[5], (int)v[6], (const int64_t*)(intptr_t)v[7],
-                         (int64_t)v[8], (int)v[9], (int)v[10], (slmt_stream_t)(intptr_t)v[11]);
-  return PyLong_FromLong(rc);
-}
-
-static PyObject* decode_paged_batched(PyObject* self, PyObject* const* args, Py_ssize_t n) {
-  (void)self;
-  long long v[22];
-  if (!g_decode) {
-    PyErr_SetString(PyExc_RuntimeError, "decode_paged_batched: library not bound");
-    return NULL;
-  }
-  if (n != 22) {
-    PyErr_SetString(PyExc_TypeError, "decode_paged_batched takes 22 arguments");
-    return NULL;
-  }
-  if (take(args, 22, v)) return NULL;
-  const int rc = g_decode((const void*)(intptr_t)v[0], (int64_t)v[1], (int64_t)v[2], (const void*)(intptr_t)v[3],
-                          (int64_t)v[4], (int)v[5], (const void*)(intptr_t)v[6], (int)v[7], (int64_t)v[8],
-                          (const int32_t*)(intptr_t)v[9], (int)v[10], (int)v[11], (int)v[12], (int)v[13],
-                          (int)v[14], (void*)(intptr_t)v[15], (int)v[16], (int64_t)v[17], (int64_t)v[18],
-                          (void*)(intptr_t)v[19], (int64_t)v[20], (slmt_stream_t)(intptr_t)v[21]);
-  return PyLong_FromLong(rc);
-}
-
+#define METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, "slmt_" #name}
 static PyMethodDef methods[] = {
-    {"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, "bind the library's entry points"},
-    {"quantize_store", (PyCFunction)(void (*)(void))quantize_store, METH_FASTCALL, "slmt_quantize_store"},
-    {"decode_paged_batched", (PyCFunction)(void (*)(void))decode_paged_batched, METH_FASTCALL,
-     "slmt_decode_paged_batched"},
+    {"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, "bind one of the library's entry points"},
+    METHOD(quantize_store),
+    METHOD(decode_paged_batched),
+    METHOD(chunk_paged),
+    METHOD(chunk_workspace_bytes),
+    METHOD(decode_per_token),
+    METHOD(decode_per_channel),
+    METHOD(prefill_per_channel),
+    METHOD(quantize_kv_per_channel),
+    METHOD(quantize_with_rulers),
     {NULL, NULL, 0, NULL}};
 
 static struct PyModuleDef module = {PyModuleDef_HEAD_INIT, "_slmt_fast", NULL, -1, methods, NULL, NULL, NULL, NULL};

@@ -91,15 +91,25 @@ def load():
         return lib
 
 
+# entry points of the METH_FASTCALL binding, without their slmt_
+_FAST_ENTRIES = ("quantize_store",
+                 "decode_paged_batched",
+                 "chunk_paged",
+                 "chunk_workspace_bytes",
+                 "decode_per_token",
+                 "decode_per_channel",
+                 "prefill_per_channel",
+                 "quantize_kv_per_channel",
+                 "quantize_with_rulers")
 _fast = None
 _fast_tried = False
 
 
 def fast():
     """The CPython METH_FASTCALL binding (kernels/_slmt_fast, built from
-    csrc/pyfast.c) bound to the loaded library's slmt_quantize_store and
-    slmt_decode_paged_batched, or None when it was not built.  It calls the
-    same entry points as the ctypes functions, with less per-call overhead."""
+    csrc/pyfast.c) bound to the loaded library's hot entry points, or None when it
+    was not built.  It calls the same entry points as the ctypes functions, with
+    less per-call overhead."""
     global _fast, _fast_tried
     if _fast_tried:
         return _fast
@@ -111,8 +121,8 @@ def fast():
             except ImportError:
                 mod = None
             if mod is not None:
-                mod.bind(ctypes.cast(lib.slmt_quantize_store, ctypes.c_void_p).value,
-                         ctypes.cast(lib.slmt_decode_paged_batched, ctypes.c_void_p).value)
+                for name in _FAST_ENTRIES:
+                    mod.bind(name, ctypes.cast(getattr(lib, "slmt_" + name), ctypes.c_void_p).value)
             _fast = mod
             _fast_tried = True
     return _fast

@@ -59,13 +59,20 @@ _fast_checked = False
 
 
 def _fastcall():
-    """The METH_FASTCALL binding of the store and batched decode (None when it
-    was not built: the ctypes functions of the same library are used then)."""
+    """The METH_FASTCALL binding of the hot entry points (None when it was not built:
+    the ctypes functions of the same library are used then)."""
     global _fast_mod, _fast_checked
     if not _fast_checked:
         _fast_mod = _native.fast()
         _fast_checked = True
     return _fast_mod
+
+
+def _entry(lib, name):
+    """Entry point slmt_<name>, through the METH_FASTCALL binding where it was built."""
+    return getattr(_fastcall() or lib, name if _fast_mod else "slmt_" + name)
+
+
 _current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
@@ -115,10 +122,13 @@ def _workspace_of(device: torch.device, need: int, stream: int) -> tuple[int, in
     return buf.data_ptr(), buf.numel()
 
 
+_no_switch = contextlib.nullcontext()
+
+
 def _on_device(dev: torch.device):
     """Make ``dev`` current for the call (no switch when it already is)."""
-    if dev.index is None or dev.index == torch.cuda.current_device():
-        return contextlib.nullcontext()
+    if dev.index is None or dev.index == _current_device():
+        return _no_switch
     return torch.cuda.device(dev)
 
 
@@ -129,17 +139,24 @@ def _require(cond: bool, msg: str) -> None:
 
 def _check_common(q, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero, phase, num_kv_heads):
     """Native-side validation (reference kernels/kv_dequant_cuda.cu:53-76)."""
-    _require(q.is_cuda, f"{phase}: q must be a CUDA tensor")
-    _require(q.dtype == torch.float16, f"{phase}: q must be fp16")
-    _require(k_packed.is_cuda and v_packed.is_cuda, f"{phase}: packed KV must be CUDA tensors")
-    _require(k_packed.dtype == torch.uint8 and v_packed.dtype == torch.uint8, f"{phase}: packed KV must be uint8")
+    # (once per layer and step: messages are formatted only when a check fails)
+    if not q.is_cuda:
+        raise RuntimeError(f"{phase}: q must be a CUDA tensor")
+    if q.dtype is not torch.float16:
+        raise RuntimeError(f"{phase}: q must be fp16")
+    if not (k_packed.is_cuda and v_packed.is_cuda):
+        raise RuntimeError(f"{phase}: packed KV must be CUDA tensors")
+    if not (k_packed.dtype is torch.uint8 and v_packed.dtype is torch.uint8):
+        raise RuntimeError(f"{phase}: packed KV must be uint8")
     for t in (k_scale, k_zero, v_scale, v_zero):
-        _require(t.is_cuda and t.dtype == torch.float16, f"{phase}: scale/zero tensors must be fp16 CUDA")
-    D, D2 = q.size(2), k_packed.size(2)
-    _require(D == 2 * D2, f"{phase}: D ({D}) must be 2 * D2 ({D2})")
-    H = q.size(0)
-    _require(num_kv_heads > 0 and H % num_kv_heads == 0,
-             f"{phase}: num_kv_heads {num_kv_heads} must divide query heads {H}")
+        if not (t.is_cuda and t.dtype is torch.float16):
+            raise RuntimeError(f"{phase}: scale/zero tensors must be fp16 CUDA")
+    H, _, D = q.shape
+    D2 = k_packed.shape[2]
+    if D != 2 * D2:
+        raise RuntimeError(f"{phase}: D ({D}) must be 2 * D2 ({D2})")
+    if not (num_kv_heads > 0 and H % num_kv_heads == 0):
+        raise RuntimeError(f"{phase}: num_kv_heads {num_kv_heads} must divide query heads {H}")
 
 
 # =============================================================================
@@ -168,7 +185,8 @@ def kv_dequant_decode_attention(
     lib = _load_native_extension()
     phase = "kv_dequant_decode"
     _check_common(q, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero, phase, num_kv_heads)
-    _require(num_kv_heads <= KV, f"{phase}: num_kv_heads {num_kv_heads} exceeds the packed KV heads {KV}")
+    if num_kv_heads > KV:
+        raise RuntimeError(f"{phase}: num_kv_heads {num_kv_heads} exceeds the packed KV heads {KV}")
     dev = q.device
     with _on_device(dev):
         out = torch.empty((H, 1, D), dtype=torch.float32, device=dev)
@@ -176,12 +194,14 @@ def kv_dequant_decode_attention(
             return out.fill_(math.nan)
         q, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero = (
             t.contiguous() for t in (q, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero))
-        ws, ws_bytes = _workspace(lib, dev, 1, H, num_kv_heads, D)
-        rc = lib.slmt_decode_per_channel(
-            _ptr(q), _ptr(k_packed), _ptr(k_scale), _ptr(k_zero), _ptr(v_packed), _ptr(v_scale),
-            _ptr(v_zero), H, KV, num_kv_heads, S, D, BLOCK_N, int(bool(use_quant)), _ptr(out),
-            ws, ws_bytes, _stream(dev))
-        _native.check(lib, rc)
+        stream = _stream(dev)
+        ws, ws_bytes = _workspace(lib, dev, 1, H, num_kv_heads, D, stream)
+        rc = _entry(lib, "decode_per_channel")(
+            q.data_ptr(), k_packed.data_ptr(), k_scale.data_ptr(), k_zero.data_ptr(), v_packed.data_ptr(),
+            v_scale.data_ptr(), v_zero.data_ptr(), H, KV, num_kv_heads, S, D, BLOCK_N, 1 if use_quant else 0,
+            out.data_ptr(), ws, ws_bytes, stream)
+        if rc:
+            _native.check(lib, rc)
     return out
 
 
@@ -221,8 +241,10 @@ def kv_dequant_prefill_attention(
     lib = _load_native_extension()
     phase = "kv_dequant_prefill"
     _check_common(q, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero, phase, num_kv_heads)
-    _require(q.dim() == 3, f"{phase}: q must be [H, M, D], got {list(q.shape)}")
-    _require(num_kv_heads <= KV, f"{phase}: num_kv_heads {num_kv_heads} exceeds the packed KV heads {KV}")
+    if q.dim() != 3:
+        raise RuntimeError(f"{phase}: q must be [H, M, D], got {list(q.shape)}")
+    if num_kv_heads > KV:
+        raise RuntimeError(f"{phase}: num_kv_heads {num_kv_heads} exceeds the packed KV heads {KV}")
     dev = q.device
     with _on_device(dev):
         out = torch.empty((H, M, D), dtype=torch.float32, device=dev)
@@ -232,12 +254,14 @@ def kv_dequant_prefill_attention(
             return out.fill_(math.nan)
         q, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero = (
             t.contiguous() for t in (q, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero))
-        ws, ws_bytes = _workspace(lib, dev, M, H, num_kv_heads, D)
-        rc = lib.slmt_prefill_per_channel(
-            _ptr(q), _ptr(k_packed), _ptr(k_scale), _ptr(k_zero), _ptr(v_packed), _ptr(v_scale),
-            _ptr(v_zero), H, KV, num_kv_heads, M, S, D, BLOCK_M, BLOCK_N, int(bool(causal)),
-            int(bool(use_quant)), _ptr(out), ws, ws_bytes, _stream(dev))
-        _native.check(lib, rc)
+        stream = _stream(dev)
+        ws, ws_bytes = _workspace(lib, dev, M, H, num_kv_heads, D, stream)
+        rc = _entry(lib, "prefill_per_channel")(
+            q.data_ptr(), k_packed.data_ptr(), k_scale.data_ptr(), k_zero.data_ptr(), v_packed.data_ptr(),
+            v_scale.data_ptr(), v_zero.data_ptr(), H, KV, num_kv_heads, M, S, D, BLOCK_M, BLOCK_N, 1 if causal else 0,
+            1 if use_quant else 0, out.data_ptr(), ws, ws_bytes, stream)
+        if rc:
+            _native.check(lib, rc)
     return out
 
 
@@ -264,14 +288,17 @@ def kv_dequant_decode_per_token_attention(
 
     lib = _load_native_extension()
     phase = "per-token decode"
-    _require(q.is_cuda and q.dtype == torch.float16, f"{phase}: q must be fp16 CUDA")
-    _require(q.dim() == 3 and q.size(1) == 1, f"{phase}: q must be [H, 1, D], got {list(q.shape)}")
-    _require(k_packed.is_cuda and v_packed.is_cuda and k_packed.dtype == torch.uint8
-             and v_packed.dtype == torch.uint8, f"{phase}: packed KV must be uint8 CUDA tensors")
+    if not (q.is_cuda and q.dtype is torch.float16):
+        raise RuntimeError(f"{phase}: q must be fp16 CUDA")
+    if not (q.dim() == 3 and q.shape[1] == 1):
+        raise RuntimeError(f"{phase}: q must be [H, 1, D], got {list(q.shape)}")
+    if not (k_packed.is_cuda and v_packed.is_cuda and k_packed.dtype is torch.uint8 and v_packed.dtype is torch.uint8):
+        raise RuntimeError(f"{phase}: packed KV must be uint8 CUDA tensors")
     for t in (k_min, k_step, v_min, v_step):
-        _require(t.is_cuda and t.dtype == torch.float16 and tuple(t.shape) == (KV, S),
-                 f"{phase}: min/step tensors must be fp16 CUDA [KV, S]")
-    _require(num_kv_heads <= KV, f"{phase}: num_kv_heads {num_kv_heads} exceeds the packed KV heads {KV}")
+        if not (t.is_cuda and t.dtype is torch.float16 and t.shape == (KV, S)):
+            raise RuntimeError(f"{phase}: min/step tensors must be fp16 CUDA [KV, S]")
+    if num_kv_heads > KV:
+        raise RuntimeError(f"{phase}: num_kv_heads {num_kv_heads} exceeds the packed KV heads {KV}")
     dev = q.device
     with _on_device(dev):
         out = torch.empty((H, 1, D), dtype=torch.float32, device=dev)
@@ -279,11 +306,14 @@ def kv_dequant_decode_per_token_attention(
             return out.fill_(math.nan)
         q, k_packed, k_min, k_step, v_packed, v_min, v_step = (
             t.contiguous() for t in (q, k_packed, k_min, k_step, v_packed, v_min, v_step))
-        ws, ws_bytes = _workspace(lib, dev, 1, H, num_kv_heads, D)
-        rc = lib.slmt_decode_per_token(
-            _ptr(q), _ptr(k_packed), _ptr(k_min), _ptr(k_step), _ptr(v_packed), _ptr(v_min),
-            _ptr(v_step), H, KV, num_kv_heads, S, D, BLOCK_N, _ptr(out), ws, ws_bytes, _stream(dev))
-        _native.check(lib, rc)
+        stream = _stream(dev)
+        ws, ws_bytes = _workspace(lib, dev, 1, H, num_kv_heads, D, stream)
+        rc = _entry(lib, "decode_per_token")(
+            q.data_ptr(), k_packed.data_ptr(), k_min.data_ptr(), k_step.data_ptr(), v_packed.data_ptr(),
+            v_min.data_ptr(), v_step.data_ptr(), H, KV, num_kv_heads, S, D, BLOCK_N, out.data_ptr(), ws, ws_bytes,
+            stream)
+        if rc:
+            _native.check(lib, rc)
     return out
 
 
@@ -448,8 +478,7 @@ def kv_dequant_decode_paged_batched(
         seq_lens = seq_lens.contiguous()
         stream = _stream(dev)
         ws, ws_bytes = _workspace(lib, dev, B, H, num_kv_heads, D, stream)
-        fast = _fastcall()
-        rc = (fast.decode_paged_batched if fast else lib.slmt_decode_paged_batched)(
+        rc = _entry(lib, "decode_paged_batched")(
             q.data_ptr(), qs[0], qs[1], kv_cache.data_ptr(), cshape[0], int(block_size),
             block_tables.data_ptr(), 64 if bt_dtype is torch.int64 else 32, bt_stride[0],
             seq_lens.data_ptr(), 0, B, H, num_kv_heads, D, out.data_ptr(),
@@ -523,11 +552,11 @@ def kv_dequant_chunk_paged(
         seq_lens, query_start_loc = seq_lens.contiguous(), query_start_loc.contiguous()
         stream = _stream(dev)
         max_seq_len = min(max(int(max_seq_len), 1), 2**31 - 1)
-        need = lib.slmt_chunk_workspace_bytes(N, R, H, num_kv_heads, D, max_seq_len)
+        need = _entry(lib, "chunk_workspace_bytes")(N, R, H, num_kv_heads, D, max_seq_len)
         if need < 0:
             raise RuntimeError(_native.last_error(lib))
         ws, ws_bytes = _workspace_of(dev, need, stream) if need else (0, 0)
-        rc = lib.slmt_chunk_paged(
+        rc = _entry(lib, "chunk_paged")(
             q.data_ptr(), qs[0], qs[1], kv_cache.data_ptr(), cshape[0], int(block_size), block_tables.data_ptr(),
             64 if bt_dtype is torch.int64 else 32, block_tables.stride(0), query_start_loc.data_ptr(),
             seq_lens.data_ptr(), max_seq_len, N, R, H, num_kv_heads, D, out.data_ptr(),
@@ -601,7 +630,7 @@ def quantize_tensor(x, scale, zero_point, bits=4, out=None):
             xs = x.stride()
         scale, zero_point = scale.contiguous(), zero_point.contiguous()
         os_ = out.stride()
-        rc = lib.slmt_quantize_with_rulers(x.data_ptr(), xs[0], xs[1], KV, S, D, scale.data_ptr(),
+        rc = _entry(lib, "quantize_with_rulers")(x.data_ptr(), xs[0], xs[1], KV, S, D, scale.data_ptr(),
                                            zero_point.data_ptr(), out.data_ptr(), os_[0], os_[1], _stream(dev))
         if rc:
             _native.check(lib, rc)
@@ -619,11 +648,13 @@ def quantize_kv(k, v):
         dev = k.device
         with _on_device(dev):
             k, v = k.contiguous(), v.contiguous()
-            kp, vp = (torch.empty((KV, S, D // 2), dtype=torch.uint8, device=dev) for _ in range(2))
-            ks, kz, vs, vz = (torch.empty((KV, D), dtype=torch.float16, device=dev) for _ in range(4))
-            rc = lib.slmt_quantize_kv_per_channel(_ptr(k), _ptr(v), KV, S, D, _ptr(kp), _ptr(ks), _ptr(kz),
-                                                  _ptr(vp), _ptr(vs), _ptr(vz), _stream(dev))
-            _native.check(lib, rc)
+            kp, vp = k.new_empty((KV, S, D // 2), dtype=torch.uint8), k.new_empty((KV, S, D // 2), dtype=torch.uint8)
+            ks, kz, vs, vz = k.new_empty((KV, D)), k.new_empty((KV, D)), k.new_empty((KV, D)), k.new_empty((KV, D))
+            rc = _entry(lib, "quantize_kv_per_channel")(
+                k.data_ptr(), v.data_ptr(), KV, S, D, kp.data_ptr(), ks.data_ptr(), kz.data_ptr(), vp.data_ptr(),
+                vs.data_ptr(), vz.data_ptr(), _stream(dev))
+            if rc:
+                _native.check(lib, rc)
         return kp, ks, kz, vp, vs, vz
     kp, ks, kz = quantize_per_channel(k)
     vp, vs, vz = quantize_per_channel(v)
