@@ -119,7 +119,12 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
     }
     return cd;
   };
-  Codes cur = load_round(0);
+  // (all rounds' loads at once: one after another each was a round trip of its own)
+  constexpr int ROUNDS = MAX_CT / NW / 16;
+  Codes codes[ROUNDS];
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r)
+    if (r == 0 || 16 * r < wn) codes[r] = load_round(r);   // uniform
 
   // q' and this lane's V rulers for the output dims 2b, 2b+1.  Every load is
   // issued first, unconditionally (rows past G re-read the last head's, the
@@ -179,10 +184,12 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
   }
 
   // ---- QK, 16 keys per round; V rows staged on the way
-  for (int r = 0; r * 16 < wn; ++r) {
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    if (16 * r >= wn) break;
     const int jw = 16 * r + t;              // key within the wave's keys
     const int j = wk0 + jw;                 // key within the chunk
-    if (r > 0) cur = load_round(r);
+    const Codes& cur = codes[r];
     uint32_t kw[2 * QW];
 #pragma unroll
     for (int i = 0; i < QW; ++i) {
@@ -259,19 +266,17 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
       vt0[h] = wave_sum(lane < wn ? e * vmin : 0.f);
     }
   }
+  if constexpr (!TOK) {
+    const int j = wk0 + lane;               // (a wave has at most 64 keys)
 #pragma unroll
-  for (int h = 0; !TOK && h < GT; ++h) {
-    float mx = -INFINITY;
-    for (int j = lane; j < wn; j += 64) mx = fmaxf(mx, sp[(wk0 + j) * 8 + h] * kscale);
-    mx = wave_max(mx);
-    float ls = 0.f;
-    for (int j = lane; j < wn; j += 64) {
-      const float e = __builtin_amdgcn_exp2f(sp[(wk0 + j) * 8 + h] * kscale - mx);
-      sp[(wk0 + j) * 8 + h] = e;
-      ls += e;
+    for (int h = 0; h < GT; ++h) {
+      const float x = lane < wn ? sp[j * 8 + h] * kscale : -INFINITY;
+      const float mx = wave_max(x);
+      const float e = lane < wn ? __builtin_amdgcn_exp2f(x - mx) : 0.f;
+      if (lane < wn) sp[j * 8 + h] = e;
+      mh[h] = mx;
+      lh[h] = wave_sum(e);
     }
-    mh[h] = mx;
-    lh[h] = wave_sum(ls);
   }
   __syncthreads();
 
@@ -280,6 +285,7 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
   float acc[GT][2];
 #pragma unroll
   for (int h = 0; h < GT; ++h) acc[h][0] = acc[h][1] = 0.f;
+#pragma unroll 4
   for (int jw = par; jw < wn; jw += step) {
     const int j = wk0 + jw;
     const uint32_t byte = vt[j * VB + b];
@@ -386,46 +392,53 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
   }
   __syncthreads();
   if (!last) return;
-  // (m, l) of every chunk at once: lane k loads chunk k's for the wave's heads;
-  // the merge coefficients exp2(m_k - M) / L go to LDS
+  // (m, l) of every chunk at once: lane k loads chunk k's for the wave's heads; the
+  // merge coefficients exp2(m_k - M) / L go to LDS.  Outputs: lane b owns dims 2b, 2b+1
+  // (head_dim 64: lanes 32-63 take the odd chunks); the partial outputs are loaded MB at
+  // a time, the first of them along with the (m, l).
   const float* kvpart = p.part + (int64_t)kv * p.nchunks * GT * (D + 2);
+  constexpr int MB = HPW == 1 ? 16 : 8;
+  float2 ov[HPW][MB];
+  auto load_parts = [&](int k, int k0) {
+    const int h = min(wave + NW * k, GT - 1);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      const int kk = min(k0 + i * step, p.nchunks - 1);   // past the last: coefficient 0
+      ov[k][i] = load_pair_agent(kvpart + ((int64_t)kk * GT + h) * (D + 2) + 2 * b);
+    }
+  };
+  float2 ml[HPW];
 #pragma unroll
   for (int k = 0; k < HPW; ++k) {
-    const int h = wave + NW * k;
-    if (h >= GT) continue;
-    float mk = -INFINITY, lk = 0.f;
-    if (lane < p.nchunks) {
-      const float2 ml = load_pair_agent(kvpart + ((int64_t)lane * GT + h) * (D + 2) + D);
-      mk = ml.x;
-      lk = ml.y;
-    }
+    const int h = min(wave + NW * k, GT - 1);
+    ml[k] = load_pair_agent(kvpart + ((int64_t)min(lane, p.nchunks - 1) * GT + h) * (D + 2) + D);
+  }
+#pragma unroll
+  for (int k = 0; k < HPW; ++k) load_parts(k, par);
+#pragma unroll
+  for (int k = 0; k < HPW; ++k) {
+    const float mk = lane < p.nchunks ? ml[k].x : -INFINITY, lk = lane < p.nchunks ? ml[k].y : 0.f;
     const float M = wave_max(mk);
     const float w = lane < p.nchunks ? __builtin_amdgcn_exp2f(mk - M) : 0.f;
     const float L = wave_sum(w * lk);
-    sw[k * NW + wave][lane] = w / L;
+    sw[k * NW + wave][lane] = w / L;        // (0 past the last chunk)
   }
   __syncthreads();
-  // outputs: lane b owns dims 2b, 2b+1 (head_dim 64: lanes 32-63 take the odd
-  // chunks); the partial outputs are loaded 8 at a time before they are used
 #pragma unroll
   for (int k = 0; k < HPW; ++k) {
     const int h = wave + NW * k;
     if (h >= GT || h >= p.G) continue;
     const float* cf = sw[k * NW + wave];
     float o0 = 0.f, o1 = 0.f;
-    for (int k0 = par; k0 < p.nchunks; k0 += 8 * step) {
-      float2 ov[8];
+    for (int k0 = par; k0 < p.nchunks; k0 += MB * step) {
+      if (k0 > par) load_parts(k, k0);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < MB; ++i) {
         const int kk = k0 + i * step;
-        ov[i] = kk < p.nchunks ? load_pair_agent(kvpart + ((int64_t)kk * GT + h) * (D + 2) + 2 * b) : make_float2(0.f, 0.f);
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int kk = k0 + i * step;
-        const float f = kk < p.nchunks ? cf[kk] : 0.f;
-        o0 = __builtin_fmaf(f, ov[i].x, o0);
-        o1 = __builtin_fmaf(f, ov[i].y, o1);
+        if (kk < p.nchunks) {
+          o0 = __builtin_fmaf(cf[kk], ov[k][i].x, o0);
+          o1 = __builtin_fmaf(cf[kk], ov[k][i].y, o1);
+        }
       }
     }
     if (D == 64) {
