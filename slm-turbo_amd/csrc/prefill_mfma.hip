@@ -25,7 +25,12 @@
 //   is o_d = s_d * (sum p (n - zr) / l - (z_d - zr_d)) in fp32.
 // * P enters in fp16 (relative 2^-11 per weight), as the decode's weights do, and
 //   the row sums l are a product of the same fp16 weights with a block of ones,
-//   so numerator and denominator see the same rounded weights.
+//   so numerator and denominator see the same rounded weights.  At head_dim 80 the
+//   weights' fp16 remainders follow in a second product: the kernel that served it
+//   before moved its maximum with every growth, so that the largest weights were exact,
+//   and one fp16 weight with the lazy maximum was less exact than that (error against 64
+//   bits 1.4e-4 there, 1.6e-4 with one product, 2.7e-6 with two; 22.3 -> 24.9 us for
+//   1000 tokens at 32 q / 8 KV heads).
 // use_quant = 0 takes the raw codes (scale 1, zero 0).  Causal row m sees keys
 // n <= m; keys past S are masked.  S = 0 yields NaN rows (0/0), as the
 // reference's kernels do.
@@ -48,8 +53,8 @@
 // dim 63 are staged evenly too, 2 bytes of K and 1 byte of V per key and thread,
 // so that no wave has more to convert than another.  Against the vector-ALU
 // kernel that took one query row at a time, us per causal prefill: 32 q / 8 KV
-// heads, 1000 tokens 480 -> 22, 4096 tokens 6277 -> 149; 8/8, 100 tokens 32.6 ->
-// 11.0 (the call's host time).  It is held to 168 VGPRs, three waves per SIMD.
+// heads, 1000 tokens 481 -> 25, 4096 tokens 6277 -> 180; 8/8, 100 tokens 32.6 ->
+// 8.5 (the call's host time).  186 VGPRs, two waves per SIMD.
 #include "slmt_internal.h"
 
 #include <type_traits>
@@ -118,7 +123,7 @@ __device__ __forceinline__ uint32_t nib_pair(uint32_t lo_all, uint32_t hi_all, i
 // Head_dim 64 is held to 128 VGPRs, four waves per SIMD (two 8-wave workgroups
 // per CU).
 template <int D, int HP>
-__global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : D == 80 ? 3 : 1))) prefill_kernel(const Params p) {
+__global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : D == 80 ? 2 : 1))) prefill_kernel(const Params p) {
   using GG = Geo<D>;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63, w = (tid >> 6) & 3;
@@ -433,11 +438,15 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
         for (int i = 0; i < 4; ++i) s[n][i] -= rebase;
       cinit = floatx4{-m_new, -m_new, -m_new, -m_new};
     }
-    half4 pb[4];
+    half4 pb[4], pr[4];
 #pragma unroll
     for (int n = 0; n < 4; ++n)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) pb[n][i] = (_Float16)__builtin_amdgcn_exp2f(s[n][i]);
+      for (int i = 0; i < 4; ++i) {
+        const float e = __builtin_amdgcn_exp2f(s[n][i]);
+        pb[n][i] = (_Float16)e;
+        if constexpr (GG::X) pr[n][i] = (_Float16)(e - (float)pb[n][i]);
+      }
     // O^T: dims 16 c + 4 grp + i.  One product covers 32 keys: the lane's 8
     // k slots are keys 32 hh + 4 grp + i and 32 hh + 16 + 4 grp + i (i < 4), the
     // same keys in the V^T operand (A) and in the weights (B = pb[2 hh], pb[2 hh + 1])
@@ -447,11 +456,19 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
       for (int hh = 0; hh < 2; ++hh) {
         const half8 b = __builtin_shufflevector(pb[2 * hh], pb[2 * hh + 1], 0, 1, 2, 3, 4, 5, 6, 7);
         o[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[c][hh], b, o[c], 0, 0, 0);
+        if constexpr (GG::X) {
+          const half8 rr = __builtin_shufflevector(pr[2 * hh], pr[2 * hh + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+          o[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[c][hh], rr, o[c], 0, 0, 0);
+        }
       }
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
       const half8 b = __builtin_shufflevector(pb[2 * hh], pb[2 * hh + 1], 0, 1, 2, 3, 4, 5, 6, 7);
       ol = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, b, ol, 0, 0, 0);
+      if constexpr (GG::X) {
+        const half8 rr = __builtin_shufflevector(pr[2 * hh], pr[2 * hh + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+        ol = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, rr, ol, 0, 0, 0);
+      }
     }
     if constexpr (ST) {
       if (t + 1 < ntiles) store(Next{});
