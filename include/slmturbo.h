@@ -153,7 +153,8 @@ int slmt_decode_paged_batched(const void* q, int64_t q_seq_stride, int64_t q_hea
  *                    tokens past query_start_loc[num_reqs] are left alone
  *   max_seq_len:     the longest of seq_lens or more; decides the split of the work only
  * Tokens that see no key produce zeros.
- * workspace: slmt_chunk_workspace_bytes of the same sizes; may be NULL where that is 0.
+ * workspace: slmt_chunk_workspace_bytes of the same sizes, 16-byte aligned, its contents of no
+ * account before or after the call; may be NULL where that is 0.
  */
 int64_t slmt_chunk_workspace_bytes(int64_t num_tokens, int num_reqs, int num_heads, int num_kv_heads, int head_dim,
                                    int max_seq_len);

@@ -547,7 +547,7 @@ int launch(const ChunkParams& p, int64_t nitems, hipStream_t stream) {
 int64_t chunk_workspace_bytes(int64_t N, int R, int H, int KV, int D, int max_seq_len) {
   const chunk::Split sp = chunk::split_of(N, R, H / KV, KV, D, max_seq_len);
   if (sp.n == 1) return 0;
-  return kWsCounterInts * 4 + chunk::items(N, R, H / KV) * KV * sp.n * chunk::BM * (D + 2) * 4;
+  return chunk::items(N, R, H / KV) * KV * sp.n * chunk::BM * (D + 2) * 4;
 }
 
 int launch_chunk(int D, ChunkParams& p, int max_seq_len, void* workspace, int64_t ws_bytes, hipStream_t stream) {
@@ -562,8 +562,9 @@ int launch_chunk(int D, ChunkParams& p, int max_seq_len, void* workspace, int64_
     const int64_t need = chunk_workspace_bytes(p.N, p.R, p.G * p.KV, p.KV, D, max_seq_len);
     if (workspace == nullptr || ws_bytes < need)
       return fail(SLMT_ERR_INVALID, "chunk: workspace of " + std::to_string(need) + " bytes required, got " + std::to_string(ws_bytes));
-    // behind the counters that the decode kernels share and leave at zero
-    p.part_o = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(workspace) + kWsCounterInts * 4);
+    if (reinterpret_cast<uintptr_t>(workspace) & 15)
+      return fail(SLMT_ERR_INVALID, "chunk: the workspace must be 16-byte aligned");
+    p.part_o = reinterpret_cast<float*>(workspace);
     p.part_ml = p.part_o + n * p.KV * sp.n * chunk::BM * D;
   }
   if (D == 64) return chunk::launch<64>(p, n, stream);

@@ -106,12 +106,7 @@ def _workspace(lib, device: torch.device, B: int, H: int, KV: int, D: int,
         if need < 0:
             raise RuntimeError(_native.last_error(lib))
         _need_cache[nkey] = need
-    return _workspace_of(device, need, _stream(device) if stream is None else stream)
-
-
-def _workspace_of(device: torch.device, need: int, stream: int) -> tuple[int, int]:
-    """The stream's scratch buffer, of ``need`` bytes or more."""
-    key = (device.index, stream)
+    key = (device.index, _stream(device) if stream is None else stream)
     buf = _ws_cache.get(key)
     if buf is None or buf.numel() < need:
         with _ws_lock:
@@ -555,13 +550,15 @@ def kv_dequant_chunk_paged(
         need = _entry(lib, "chunk_workspace_bytes")(N, R, H, num_kv_heads, D, max_seq_len)
         if need < 0:
             raise RuntimeError(_native.last_error(lib))
-        ws, ws_bytes = _workspace_of(dev, need, stream) if need else (0, 0)
+        # (the partials of this call alone, in stream order like any tensor: the streams' kept
+        # buffers, which captured graphs may hold, are not grown for them)
+        ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
         rc = _entry(lib, "chunk_paged")(
             q.data_ptr(), qs[0], qs[1], kv_cache.data_ptr(), cshape[0], int(block_size), block_tables.data_ptr(),
             64 if bt_dtype is torch.int64 else 32, block_tables.stride(0), query_start_loc.data_ptr(),
             seq_lens.data_ptr(), max_seq_len, N, R, H, num_kv_heads, D, out.data_ptr(),
             _native.OUT_F16 if out_dtype is torch.float16 else _native.OUT_F32, out_stride[0], out_stride[1],
-            ws, ws_bytes, stream)
+            ws.data_ptr() if need else 0, need, stream)
         if rc:
             _native.check(lib, rc)
     return out
