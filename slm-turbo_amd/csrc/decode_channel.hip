@@ -467,18 +467,21 @@ int launch_decode_split(bool per_token, const void* q, const void* kp, const voi
   if (G < 1 || G > 8 || S < 1) return SLMT_ERR_UNSUPPORTED;
   const int KV = H / G;
   // chunk size: workgroups of four waves, each wave a multiple of 16 keys; the
-  // smallest power of two from 64 keys per workgroup that gives at most 32
-  // chunks per KV head (the merge reads every chunk's partials) and at most
-  // 256 workgroups; past 16384 keys the general kernel takes over (64 chunks)
+  // smallest power of two from 64 keys per workgroup that gives at most 16 (64 keys,
+  // but for 8 head slots of 128 dims, whose waves have the most to do per key) or 32
+  // chunks per KV head (the merge reads every chunk's partials) and at most 256
+  // workgroups; past 16384 keys the general kernel takes over (64 chunks).  us at 64,
+  // 128 and 256 keys: 700 tokens, 32 q / 4 KV heads, 64 dims 8.4, 9.3, 11.4; 1500 10.3,
+  // 9.6, 11.5; 3000 13.2, 11.6, 11.9; 1500 tokens, 12/2 heads, 128 dims 12.0, 12.8, 16.2.
+  const int GT = G <= 1 ? 1 : G <= 2 ? 2 : G <= 4 ? 4 : 8;
   int ct = 64;
   while (ct < chan::MAX_CT) {
-    const int n = (S + ct - 1) / ct;
-    if (n <= 32 && n * KV <= 256) break;
+    const int n = (S + ct - 1) / ct, most = ct == 64 && !(D == 128 && GT == 8) ? 16 : 32;
+    if (n <= most && n * KV <= 256) break;
     ct *= 2;
   }
   const int nchunks = (S + ct - 1) / ct;
   if (nchunks > 64) return SLMT_ERR_UNSUPPORTED;
-  const int GT = G <= 1 ? 1 : G <= 2 ? 2 : G <= 4 ? 4 : 8;
   const int64_t part_bytes = (int64_t)KV * nchunks * GT * (D + 2) * 4;
   const int64_t part_off = kWsCounterInts * 4;
   if (nchunks > 1 && (workspace == nullptr || ws_bytes < part_off + part_bytes || KV > kWsCounterInts))
