@@ -350,6 +350,7 @@ def test_store_row_remainders_and_special_values(N, KV, D):
     (24, 3, 64, 16, [5000], [24]),
     (5, 5, 128, 128, [200, 150], [130, 20]),
     (64, 1, 64, 16, [70, 3], [3, 1]),
+    (8, 2, 64, 16, [20 + 3 * i for i in range(140)], [i % 4 for i in range(140)]),   # three scans of 64 requests
 ])
 def test_chunk_matches_oracle(H, KV, D, bs, lens, qlens):
     """fp32 results: codes and query are exact operands, weights carry ~22 bits, so
