@@ -193,16 +193,15 @@ class PackedKVAttentionMixin:
         72 / 75 against 82 / 105, 64 of 8000 254 / 243 / 280 against 209 / 377 / 548; 32
         / 4 heads, 64 dims, 64 of 8000 90 / 103 / 191 against 118 / 201 / 286."""
         block_size, num_kv_heads = kv_cache.shape[1], kv_cache.shape[2]
-        R = attn_metadata.query_start_loc.numel() - 1
+        lens, table, qsl = attn_metadata.seq_lens, attn_metadata.block_table, attn_metadata.query_start_loc
+        R = min(qsl.numel() - 1, lens.shape[0], table.shape[0])    # (padding entries hold no tokens)
         most = int(attn_metadata.max_seq_len)
         if (query.is_cuda and 16 <= block_size <= 1024 and block_size & (block_size - 1) == 0
                 and (N * most <= 200_000 or 2 * N >= (3 if self.head_size == 64 else 10) * R)):
             kd = self._slm_kernels()
-            seq_lens, tables = _first(attn_metadata.seq_lens, R), _first(attn_metadata.block_table, R)
-            qsl = attn_metadata.query_start_loc
             self._into_output(output, N, lambda out, dtype: kd.kv_dequant_chunk_paged(
-                query, kv_cache, tables, _int32(seq_lens), _int32(qsl), most, block_size, num_kv_heads, out=out,
-                out_dtype=dtype))
+                query, kv_cache, _first(table, R), _int32(_first(lens, R)), _int32(_first(qsl, R + 1)), most, block_size,
+                num_kv_heads, out=out, out_dtype=dtype))
             return
         qsl = attn_metadata.query_start_loc.to(torch.int64)       # [R+1]
         R = qsl.numel() - 1
