@@ -29,7 +29,7 @@
 //   weights' fp16 remainders follow in a second product: the kernel that served it
 //   before moved its maximum with every growth, so that the largest weights were exact,
 //   and one fp16 weight with the lazy maximum was less exact than that (error against 64
-//   bits 1.4e-4 there, 1.6e-4 with one product, 2.7e-6 with two; 22.3 -> 24.9 us for
+//   bits 1.4e-4 there, 1.6e-4 with one product, 2.8e-7 with two; 22.3 -> 24.9 us for
 //   1000 tokens at 32 q / 8 KV heads).
 // use_quant = 0 takes the raw codes (scale 1, zero 0).  Causal row m sees keys
 // n <= m; keys past S are masked.  S = 0 yields NaN rows (0/0), as the
@@ -102,6 +102,12 @@ struct Geo {
   static constexpr int KW = D / 64;         // 8-byte K words per staging thread (K: 4 threads per key)
   static constexpr int VW = D / 64;         // V dwords per key per staging thread (V: 8 threads per key pair)
   static constexpr bool X = D == 80;        // 16 dims more: 2 bytes of K, 1 of V per key and thread
+  // Head_dim 80: K enters as code 2^-10 and the query column times 2^10, which costs
+  // nothing and keeps the column's low halves out of fp16's subnormals (below 1/8 of
+  // x they had fewer than 11 bits; now below 2^-13).
+  static constexpr float QUP = X ? 1024.0f : 1.0f;
+  static constexpr uint32_t KBITS = X ? 0x3C003C00u : 0x64006400u;   // 1 + n 2^-10; 1024 + n
+  static constexpr float KZERO = X ? 1.0f : 1024.0f;
 };
 
 __device__ __forceinline__ float hf(uint16_t h) { return h2f(h); }
@@ -112,9 +118,9 @@ __device__ __forceinline__ float hf(uint16_t h) { return h2f(h); }
 // are contiguous.  Even keys stay even: a key pair stays one 4-byte word.
 __device__ __forceinline__ int vpos(int k) { return (k & 32) | ((k & 12) << 1) | ((k & 16) >> 2) | (k & 3); }
 
-// fp16 pairs (1024 + low nibble, 1024 + high nibble) of byte i of x, minus zc
-__device__ __forceinline__ uint32_t nib_pair(uint32_t lo_all, uint32_t hi_all, int i, half2v zc) {
-  const uint32_t w = __builtin_amdgcn_perm(hi_all, lo_all, 0x0C000C00u | ((4u + i) << 16) | (uint32_t)i) | 0x64006400u;
+// fp16 pairs (low nibble, high nibble) of byte i of x under the bits of `one`, minus zc
+__device__ __forceinline__ uint32_t nib_pair(uint32_t lo_all, uint32_t hi_all, int i, uint32_t one, half2v zc) {
+  const uint32_t w = __builtin_amdgcn_perm(hi_all, lo_all, 0x0C000C00u | ((4u + i) << 16) | (uint32_t)i) | one;
   const half2v r = __builtin_bit_cast(half2v, w) - zc;
   return __builtin_bit_cast(uint32_t, r);
 }
@@ -143,17 +149,21 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
   const bool quant = p.use_quant != 0;
 
   // ---- the lane's query column, scaled per channel and by log2(e) / sqrt(D) (so
-  // the scores come out as base-2 logits), split hi / lo (B operand of S^T)
-  const float sc = 1.4426950408889634f * __builtin_amdgcn_rsqf((float)D);
+  // the scores come out as base-2 logits), split hi / lo (B operand of S^T).  A column
+  // that does not fit fp16 (it would be infinity minus infinity) is read again and enters
+  // at a power of two of its own; its wave then takes the loop that multiplies each score
+  // by `unit` (`wide`; the lane's unit waits in LDS).
+  const float sc = 1.4426950408889634f * __builtin_amdgcn_rsqf((float)D) * GG::QUP;
   constexpr int QB = GG::QB;
   half8 qh[QB], ql[QB];
-  {
+  auto column = [&](auto scaled, int ex) {                    // the lane's part times 2^ex; returns its largest value
     // The rulers are read whether or not use_quant is set (the pointers are
     // always valid), so that every load of the prologue is issued before the
     // first wait; under a per-element branch each load waited for the previous.
     const uint16_t* qrow = p.q + ((int64_t)h * p.M + mq) * D;
     uint4 raw[QB];
     uint16_t ksr[QB][8];
+    float amax = 0.f;
 #pragma unroll
     for (int j = 0; j < QB; ++j) {
       const int d0 = min(32 * j + 8 * grp, D - 8);   // head_dim 80, past its dims: re-read, zeroed below
@@ -169,12 +179,20 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
         float x = hf((uint16_t)(wds[e >> 1] >> (16 * (e & 1)))) * sc;
         x *= quant ? hf(ksr[j][e]) : 1.0f;
         if (32 * j + 8 * grp >= D) x = 0.f;
+        amax = fmaxf(amax, fabsf(x));
+        if constexpr (decltype(scaled)::value) x = __builtin_amdgcn_ldexpf(x, ex);
+        // (rounded to fp32 once for both uses: the compiler otherwise joins the products
+        // with one conversion and not the other, and where these differ the low half is
+        // off by an fp16 ulp: error at head_dim 80, 1000 tokens, 4.8e-6 -> 2.8e-7)
+        asm("" : "+v"(x));
         const _Float16 hi = (_Float16)x;
         qh[j][e] = hi;
         ql[j][e] = (_Float16)(x - (float)hi);
       }
     }
-  }
+    return amax;
+  };
+  float amax = column(std::false_type{}, 0);
 
   // ---- staging roles
   // K: thread (key kk, quarter ku): dims D/4 * ku .. + D/4 - 1.  Staging wave v
@@ -182,7 +200,7 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
   // the lanes of a quarter write consecutive rows, and the wave's loads cover
   // its 16 keys' codes contiguously.
   const int kk = (tid & 15) + 16 * ((tid >> 6) & 3), ku = (tid >> 4) & 3;
-  const half2v kzc = half2v{(_Float16)1024.0f, (_Float16)1024.0f};
+  const half2v kzc = half2v{(_Float16)GG::KZERO, (_Float16)GG::KZERO};
   // V: thread (key pair vk, byte group vb (+ 8)): dims 8 vb .. 8 vb + 7, each with
   // 1024 + its rounded zero point.  Staging wave v takes all 32 key pairs of the
   // tile for byte groups 2 v and 2 v + 1 (lane l: key pair l & 31, byte group
@@ -278,7 +296,7 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
           const int pi = 8 * i + 4 * hw + b;     // dim pair index within the thread's quarter
-          kw[pi] = nib_pair(lo, hi, b, kzc);
+          kw[pi] = nib_pair(lo, hi, b, GG::KBITS, kzc);
         }
       }
     }
@@ -287,7 +305,7 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
     for (int i = 0; i < 2 * GG::KW; ++i) kd[i] = make_uint4(kw[4 * i], kw[4 * i + 1], kw[4 * i + 2], kw[4 * i + 3]);
     if constexpr (GG::X) {
       const uint32_t lo = kxx[sl] & 0x0F0Fu, hi = (kxx[sl] >> 4) & 0x0F0Fu;
-      *reinterpret_cast<uint2*>(Ks + kk * GG::KROW + 128 + 8 * ku) = make_uint2(nib_pair(lo, hi, 0, kzc), nib_pair(lo, hi, 1, kzc));
+      *reinterpret_cast<uint2*>(Ks + kk * GG::KROW + 128 + 8 * ku) = make_uint2(nib_pair(lo, hi, 0, GG::KBITS, kzc), nib_pair(lo, hi, 1, GG::KBITS, kzc));
       // the two keys' bytes: low nibbles are dim 64 + 2 vb, high nibbles the next
       const uint32_t b2 = vxx[sl][0] | (vxx[sl][1] << 16);
       const half2v ze = __builtin_shufflevector(vzx, vzx, 0, 0), zo = __builtin_shufflevector(vzx, vzx, 1, 1);
@@ -326,7 +344,7 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
   // (0 before the first tile), so the scores come out of the matrix cores as
   // base-2 logits relative to it and need no subtraction per score.  The C
   // operand is this persistent register block, rewritten only when the maximum
-  // moves; it also is the running maximum's only copy.
+  // moves; it also is the running maximum's only copy (in the products' units).
   floatx4 cinit = floatx4{0.f, 0.f, 0.f, 0.f};
 
   using S0 = std::integral_constant<int, 0>;
@@ -348,11 +366,25 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
     load(min(1, ntiles - 1), S1{});
     store(S0{});
   }
+  // (tested here, behind the tile loads: ahead of them the test made them wait for the
+  // query, 2 % of a long prefill)
+  const bool wide = __builtin_amdgcn_ballot_w64(amax >= 65520.0f) != 0;   // uniform over the wave
+  float* const unit = reinterpret_cast<float*>(smem + 2 * GG::STAGE) + tid;
+  if (wide) {
+    float a, b;                                               // over the four lane groups that hold the column
+    swap16(amax, a, b);
+    amax = fmaxf(a, b);
+    swap32(amax, a, b);
+    amax = fmaxf(a, b);
+    const int ex = amax >= 65520.0f ? 15 - __builtin_amdgcn_frexp_expf(amax) : 0;
+    *unit = __builtin_amdgcn_ldexpf(1.0f, -ex);               // (read by this lane alone)
+    column(std::true_type{}, ex);
+  }
   __syncthreads();
   // iteration t: tile t is in LDS stage t % 2, tile t + 1 in register slot (t + 1) % 2
-  auto iteration = [&](int t, auto slot, auto role) {
+  auto iteration = [&](int t, auto slot, auto role, auto range) {
     constexpr int sl = decltype(slot)::value;
-    constexpr bool ST = decltype(role)::value;
+    constexpr bool ST = decltype(role)::value, WIDE = decltype(range)::value;
     using Next = std::integral_constant<int, sl ^ 1>;
     if constexpr (ST) load(min(t + 2, ntiles - 1), slot);   // slot sl held tile t, already in LDS
     const uint8_t* Ks = smem + sl * GG::STAGE;
@@ -376,6 +408,11 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
         s[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[n][j], qh[j], s[n], 0, 0, 0);
         s[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[n][j], ql[j], s[n], 0, 0, 0);
       }
+    }
+    if constexpr (WIDE) {
+      const float u = *unit;
+#pragma unroll
+      for (int n = 0; n < 4; ++n) s[n] *= u;
     }
     // The V^T operands of the tile, read now so that their LDS latency hides
     // behind the softmax: dims 16 c + col, keys 32 hh + 4 grp + i and
@@ -417,10 +454,10 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
     // -inf, 1 where a column's maximum did not grow).  Key 0 is visible to every
     // row, so the first tile sets a finite maximum.  The test runs on the lane's
     // own 16 scores (some lane exceeds iff some column does); the column maximum
-    // across the four lane groups is formed only when it fires.  s holds
-    // logit - off, and off = m_run once m_run is finite.
-    const float off = -cinit[0];
-    const float m_run = t == 0 ? -INFINITY : off;
+    // across the four lane groups is formed only when it fires.  The scores move by
+    // the growth itself and not by the difference of two maxima: at logits of 2^27
+    // and more that difference is off by more than the weights' range, and the
+    // largest weight was 0 or infinite.
     if (__builtin_amdgcn_ballot_w64(tmax > (t == 0 ? -INFINITY : 8.0f))) {
       // across the four lane groups (rows of 16 lanes) that hold the column
       float a, b;
@@ -428,17 +465,17 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
       tmax = fmaxf(a, b);
       swap32(tmax, a, b);
       tmax = fmaxf(a, b);
-      const float m_new = fmaxf(m_run, tmax + off);
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      const float up = t == 0 ? tmax : fmaxf(tmax, 0.f);
+      const float alpha = t == 0 ? 0.f : __builtin_amdgcn_exp2f(-up);
       ol *= alpha;
 #pragma unroll
       for (int c = 0; c < D / 16; ++c) o[c] *= alpha;
-      const float rebase = m_new - off;
 #pragma unroll
       for (int n = 0; n < 4; ++n)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[n][i] -= rebase;
-      cinit = floatx4{-m_new, -m_new, -m_new, -m_new};
+        for (int i = 0; i < 4; ++i) s[n][i] -= up;
+      const float c = cinit[0] - (WIDE ? up / *unit : up);   // (a power of two: exact)
+      cinit = floatx4{c, c, c, c};
     }
     half4 pb[4], pr[4];
 #pragma unroll
@@ -477,14 +514,16 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
     }
     __syncthreads();
   };
-  auto run = [&](auto role) {
+  auto run = [&](auto role, auto range) {
     for (int t = 0; t < ntiles; t += 2) {
-      iteration(t, S0{}, role);
-      if (t + 1 < ntiles) iteration(t + 1, S1{}, role);
+      iteration(t, S0{}, role, range);
+      if (t + 1 < ntiles) iteration(t + 1, S1{}, role, range);
     }
   };
-  if (stager) run(std::true_type{});
-  else run(std::false_type{});
+  using T = std::true_type;
+  using F = std::false_type;
+  if (HP == 1 || stager) wide ? run(T{}, T{}) : run(T{}, F{});
+  else wide ? run(F{}, T{}) : run(F{}, F{});
 
   // every row of the ones product holds the column's whole sum
   const float rl = 1.0f / ol[0];
@@ -534,13 +573,13 @@ template <int D, int HP>
 int launch_hp(Params p, hipStream_t stream) {
   static const bool lds_ok = [] {   // above 64 KB of LDS (head_dim 128) needs the attribute
     return hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_kernel<D, HP>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, Geo<D>::LDS) == hipSuccess;
+                               hipFuncAttributeMaxDynamicSharedMemorySize, Geo<D>::LDS + 1024 * HP) == hipSuccess;
   }();
   if (!lds_ok) return fail(SLMT_ERR_HIP, "prefill: could not grant the kernel its LDS");
   const int grid = p.qblocks * (p.H / HP);
   const int cus = device_cu_count();
   p.paired = HP == 1 && p.causal && 8 * grid >= 11 * cus && grid <= 2 * cus;
-  hipLaunchKernelGGL((prefill_kernel<D, HP>), dim3(grid), dim3(256 * HP), Geo<D>::LDS, stream, p);
+  hipLaunchKernelGGL((prefill_kernel<D, HP>), dim3(grid), dim3(256 * HP), Geo<D>::LDS + 1024 * HP, stream, p);
   return check_launch("prefill");
 }
 

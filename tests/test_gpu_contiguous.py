@@ -421,3 +421,44 @@ def test_decode_split_per_token_and_head_dim_80(H, KV, D, S):
         c = [x.to(dev) for x in (packed[0], scale[0], zero[0], packed[1], scale[1], zero[1])]
         out = kd.kv_dequant_decode_attention(q.to(dev), *c)
         assert_close(out.cpu().numpy(), ref, atol=1e-5 * np.abs(ref).max(), rtol=0, what="per-channel split, head_dim 80")
+
+
+# Columns of q * k_scale past fp16's largest number beside ordinary ones of the same
+# 16-row block: the pairs that hold a column carry a power of two of its own.
+@pytest.mark.parametrize("H,KV,D", [(4, 2, 64), (4, 2, 80), (4, 2, 128), (3, 3, 80)])
+@pytest.mark.parametrize("M,S,causal,quant", [(150, 150, True, True), (17, 70, False, True), (33, 33, True, False)])
+def test_prefill_wide_range_queries(H, KV, D, M, S, causal, quant):
+    g = torch.Generator().manual_seed(D + M)
+    q = torch.randn(H, M, D, generator=g)
+    q[:, ::3] *= 100.0 if quant else 6000.0
+    q[:, 1::3] *= 1e-3 if quant else 1.0
+    q[0, M - 1] = 65504.0
+    q = q.clamp(-65504, 65504).half()
+    packed = torch.randint(0, 256, (2, KV, S, D // 2), generator=g, dtype=torch.uint8)
+    scale = (torch.rand(2, KV, D, generator=g) * 0.4 + 0.05).half()
+    scale[0, 0] = 5000.0 * (1 + scale[0, 0])
+    zero = torch.randint(0, 16, (2, KV, D), generator=g).half()
+    t = (packed[0], scale[0], zero[0], packed[1], scale[1], zero[1])
+    out = _kd().kv_dequant_prefill_attention(q.to(DEV), *[x.to(DEV) for x in t], causal=causal, use_quant=quant)
+    ref = oa.prefill_per_channel(q.numpy(), *[x.numpy() for x in t], causal=causal, use_quant=quant)
+    assert np.isfinite(ref).all()
+    assert_close(out.cpu().numpy(), ref, what=f"D={D} causal={causal} quant={quant}")
+
+
+# Head_dim 80 holds the query column in 22 bits and its weights too, so what is left is
+# fp32 rounding: logits of up to about 10 (0.5 for the small column) that are off by a
+# few 2^-24 of their size, 4 * 10 * 2^-24 = 2.4e-6 at the most and less on average.
+@pytest.mark.parametrize("ks,qf,bound", [(0.47, 1.0, 1e-6), (0.05, 0.05, 5e-7)])
+def test_prefill_head_dim_80_precision(ks, qf, bound):
+    g = torch.Generator().manual_seed(5)
+    H, KV, D, S = 8, 2, 80, 600
+    q = (torch.randn(H, S, D, generator=g) * qf).half()
+    packed = torch.randint(0, 256, (2, KV, S, D // 2), generator=g, dtype=torch.uint8)
+    scale = (torch.rand(2, KV, D, generator=g) * 0.4 + 0.05).half()
+    scale[0] *= ks / 0.25
+    zero = torch.randint(0, 16, (2, KV, D), generator=g).half()
+    t = (packed[0], scale[0], zero[0], packed[1], scale[1], zero[1])
+    out = _kd().kv_dequant_prefill_attention(q.to(DEV), *[x.to(DEV) for x in t]).cpu().numpy().astype(np.float64)
+    ref = oa.prefill_per_channel(q.numpy(), *[x.numpy() for x in t])
+    err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+    assert err <= bound, err
