@@ -16,7 +16,9 @@
 //     key codes with every head in fp32 and the quad adds the quarters.  The
 //     zero point's term sum_d q'_d k_zero_d is the same for every key of a head,
 //     so it cancels in the softmax and is never formed; the rest is exact fp32
-//     on exact integer codes;
+//     on exact integer codes.  (A zero point that is NaN or infinite, as the quantizer
+//     leaves for a channel whose scale underflowed, makes the head NaN at head_dim 80,
+//     as the general kernel did there; at 64 and 128 it has always gone unseen.)
 //   * softmax over the wave's keys per head (wave reductions), weights to LDS;
 //   * PV: lane = V byte (two dims): sum over the wave's keys of p * code;
 //   * the four waves' (m, l, acc) are combined by log-sum-exp in LDS, wave w
@@ -44,7 +46,7 @@ struct Params {
   const uint16_t* q;                        // [H, 1, D] fp16
   const uint8_t* kp;                        // [KV_t, S, D/2]
   const uint8_t* vp;
-  const uint16_t *ks, *vs, *vz;             // per channel: [KV_t, D] fp16
+  const uint16_t *ks, *kz, *vs, *vz;        // per channel: [KV_t, D] fp16
   const uint16_t *tr[4];                    // per token: K min and step, V min and step, [KV_t, S] fp16
   float* out;                               // [H, 1, D]
   float* part;                              // [KV][nchunks][GT][D + 2] partials
@@ -133,13 +135,14 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
   const int b = min(lane % NB, VB - 1), par = lane / NB, step = 64 / NB;
   const bool writes = lane < min(NB, VB);
   constexpr int QN = (GT * D + 64 * NW - 1) / (64 * NW);   // q' elements per thread
-  uint16_t qraw[QN], kraw[QN], vsr[2], vzw[2], tr[4];
+  uint16_t qraw[QN], kraw[QN], zraw[QN], vsr[2], vzw[2], tr[4];
 #pragma unroll
   for (int u = 0; u < QN; ++u) {
     const int i = min(tid + u * 64 * NW, GT * D - 1);
     const int h = min(i / D, p.G - 1), d = i % D;
     qraw[u] = p.q[(int64_t)(h0 + h) * D + d];
     if constexpr (!TOK) kraw[u] = p.ks[(int64_t)kv * D + d];
+    if constexpr (!TOK && X) zraw[u] = p.kz[(int64_t)kv * D + d];
   }
   if constexpr (TOK) {
     // rulers of the wave's key `lane` (a wave has at most 64), for the softmax
@@ -167,6 +170,8 @@ __global__ void __launch_bounds__(64 * NW) split_kernel(const Params p) {
     if (i < GT * D) {
       float x = h2f(qraw[u]);
       if constexpr (!TOK) x *= quant ? h2f(kraw[u]) : 1.f;
+      // (head_dim 80: a zero point that is no number does not cancel, and the head is NaN)
+      if constexpr (!TOK && X) x = quant ? x + x * h2f(zraw[u]) * 0.f : x;
       qs[i] = i / D < p.G ? x : 0.f;
     }
   }
@@ -494,8 +499,9 @@ int launch_decode_split(bool per_token, const void* q, const void* kp, const voi
   for (int i = 0; i < 4; ++i) r[i] = reinterpret_cast<const uint16_t*>(rulers[i]);
   if (per_token) {
     for (int i = 0; i < 4; ++i) p.tr[i] = r[i];
-  } else {   // the key zero point cancels in the softmax
+  } else {
     p.ks = r[0];
+    p.kz = r[1];
     p.vs = r[2];
     p.vz = r[3];
   }

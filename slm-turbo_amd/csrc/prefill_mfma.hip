@@ -162,14 +162,17 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
     // first wait; under a per-element branch each load waited for the previous.
     const uint16_t* qrow = p.q + ((int64_t)h * p.M + mq) * D;
     uint4 raw[QB];
-    uint16_t ksr[QB][8];
+    uint16_t ksr[QB][8], kzr[QB][8];
     float amax = 0.f;
 #pragma unroll
     for (int j = 0; j < QB; ++j) {
       const int d0 = min(32 * j + 8 * grp, D - 8);   // head_dim 80, past its dims: re-read, zeroed below
       raw[j] = *reinterpret_cast<const uint4*>(qrow + d0);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) ksr[j][e] = p.ks[(int64_t)kv * D + d0 + e];
+      for (int e = 0; e < 8; ++e) {
+        ksr[j][e] = p.ks[(int64_t)kv * D + d0 + e];
+        if constexpr (GG::X) kzr[j][e] = p.kz[(int64_t)kv * D + d0 + e];
+      }
     }
 #pragma unroll
     for (int j = 0; j < QB; ++j) {
@@ -178,6 +181,9 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
       for (int e = 0; e < 8; ++e) {
         float x = hf((uint16_t)(wds[e >> 1] >> (16 * (e & 1)))) * sc;
         x *= quant ? hf(ksr[j][e]) : 1.0f;
+        // head_dim 80: K zero points that are no numbers make the head's rows NaN, as in the
+        // formula that the zero point cancels in
+        if constexpr (GG::X) x = quant ? x + x * hf(kzr[j][e]) * 0.f : x;
         if (32 * j + 8 * grp >= D) x = 0.f;
         amax = fmaxf(amax, fabsf(x));
         if constexpr (decltype(scaled)::value) x = __builtin_amdgcn_ldexpf(x, ex);

@@ -462,3 +462,21 @@ def test_prefill_head_dim_80_precision(ks, qf, bound):
     ref = oa.prefill_per_channel(q.numpy(), *[x.numpy() for x in t])
     err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
     assert err <= bound, err
+
+
+# A channel whose scale underflows to 0 with the minimum 0 has the zero point NaN
+# (0 / 0), and the formula makes every output of its KV head NaN, as head_dim 80 does.
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_head_dim_80_zero_points_that_are_no_numbers(bad):
+    H, KV, D, S = 4, 2, 80, 130
+    q, t = _pc_inputs(5, H, KV, S, D, False)
+    t[2][0, 77] = bad                                                    # the K zero point of the first KV head
+    dev = [x.to(DEV) for x in t]
+    qs = torch.randn(H, 40, D, generator=torch.Generator().manual_seed(1)).half()
+    for out, ref in [(_kd().kv_dequant_decode_attention(q.to(DEV), *dev), oa.decode_per_channel(q.numpy(), *[x.numpy() for x in t])),
+                     (_kd().kv_dequant_prefill_attention(qs.to(DEV), *dev), oa.prefill_per_channel(qs.numpy(), *[x.numpy() for x in t]))]:
+        out = out.cpu().numpy()
+        assert np.isnan(out[:H // KV]).all() and np.isnan(ref[:H // KV]).all()
+        assert_close(out[H // KV:], ref[H // KV:], what=f"zero point {bad}, the other KV head")
+    raw = _kd().kv_dequant_decode_attention(q.to(DEV), *dev, use_quant=False)
+    assert torch.isfinite(raw).all()                                     # the raw codes need no ruler
