@@ -511,16 +511,28 @@ struct Split {
 // to 64 requests of 600 to 32000 tokens; us, one part, the rule's and the best: 500 tokens on
 // 2000, 32 q / 4 KV heads, 64 dims 52.5, 41.3, 39.7; 512 on 32000, 32 / 8 heads, 128
 // dims 1110, 585, 579.
+// The partials are memory that the caller has to find in the middle of a step (they are
+// allocated with the call), so a split has to give a twentieth at least and its partials
+// stay within kPartBytes: by the time alone 8192 tokens of 4 requests at 131072 keys, 64 /
+// 8 heads of 128 dims, took 783 MiB for 2.5 %, and of 8 requests at 16384, 32 / 8 heads,
+// 264 MiB to be slower (4371 us, 4283 in one part).
+constexpr int64_t kPartBytes = int64_t(128) << 20;
+int64_t part_bytes(int64_t N, int R, int G, int KV, int D) { return items(N, R, G) * KV * BM * (D + 2) * 4; }
+
 Split split_of(int64_t N, int R, int G, int KV, int D, int max_seq_len) {
   // (about as many workgroups as the requests fill: their last blocks are half full)
   const int64_t wgs = std::max<int64_t>(1, std::max<int64_t>(std::min<int64_t>(R, N), N * G / BM + R / 2) * KV);
-  const int64_t slots = (int64_t)std::max(1, device_cu_count()) * (D == 64 ? 21 : 14) / 8;
+  const int cus = device_cu_count();
+  const int64_t slots = (int64_t)(cus > 0 ? cus : 256) * (D == 64 ? 21 : 14) / 8;   // (sizes asked for without a device: the MI355X)
+  const int64_t part = std::max<int64_t>(1, part_bytes(N, R, G, KV, D));
   const int tiles = std::max(1, (int)(((int64_t)std::max(max_seq_len, 1) + BN - 1) / BN));
+  const int most = (int)std::min<int64_t>(std::min(32, std::max(1, tiles / 2)), kPartBytes / part);
   int best = 1;
-  int64_t least = INT64_MAX;
-  for (int n = 1; n <= std::min(32, std::max(1, tiles / 2)); ++n) {
+  int64_t one = 0, least = 0;
+  for (int n = 1; n <= std::max(1, most); ++n) {
     const int64_t time = ((wgs * n + slots - 1) / slots) * ((tiles + n - 1) / n + 3) + (n > 1 ? wgs * n / 90 : 0);
-    if (time < least) {
+    if (n == 1) one = least = time;
+    if (time < least && 20 * time <= 19 * one) {
       least = time;
       best = n;
     }
@@ -547,7 +559,7 @@ int launch(const ChunkParams& p, int64_t nitems, hipStream_t stream) {
 int64_t chunk_workspace_bytes(int64_t N, int R, int H, int KV, int D, int max_seq_len) {
   const chunk::Split sp = chunk::split_of(N, R, H / KV, KV, D, max_seq_len);
   if (sp.n == 1) return 0;
-  return chunk::items(N, R, H / KV) * KV * sp.n * chunk::BM * (D + 2) * 4;
+  return chunk::part_bytes(N, R, H / KV, KV, D) * sp.n;
 }
 
 int launch_chunk(int D, ChunkParams& p, int max_seq_len, void* workspace, int64_t ws_bytes, hipStream_t stream) {

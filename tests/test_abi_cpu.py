@@ -67,6 +67,25 @@ def test_version_and_workspace_sizes(lib):
     assert counters * 4 <= lib.slmt_attention_workspace_bytes(0, 32, 8, 128) <= a <= b
 
 
+# A chunk step allocates its partials with the call, beside a cache that has the memory:
+# they stay within 128 MiB, and a split that gives little is not made.
+@pytest.mark.parametrize("N,R,H,KV,D,longest,split", [
+    (8192, 4, 64, 8, 128, 131072, False), (8192, 8, 32, 8, 128, 16384, False), (16128, 32, 64, 8, 128, 131072, False),
+    (512, 13, 32, 4, 64, 2000, True), (512, 1, 32, 8, 128, 32000, True), (2048, 1, 32, 8, 128, 32000, True),
+    (1, 1, 8, 8, 80, 2**31 - 1, True), (1, 1, 8, 8, 80, 64, False), (0, 0, 8, 8, 64, 1, False)])
+def test_chunk_partials_stay_small(lib, N, R, H, KV, D, longest, split):
+    need = lib.slmt_chunk_workspace_bytes(N, R, H, KV, D, longest)
+    assert (0 < need if split else need == 0) and need <= 128 << 20
+
+
+def test_chunk_partials_stay_small_over_the_range(lib):
+    for N in (1, 17, 512, 2048, 16384, 100000):
+        for R in (1, 7, 64):
+            for H, KV in ((8, 8), (32, 4), (64, 8), (128, 1)):
+                for longest in (100, 4096, 131072):
+                    assert 0 <= lib.slmt_chunk_workspace_bytes(N, R, H, KV, 128, longest) <= 128 << 20
+
+
 def _paged_args(**kw):
     a = dict(q=16, qs=4096, qh=128, cache=16, nb=4, bs=16, bt=16, bits=32, bts=4, sl=None, fixed=5,
              B=1, H=32, KV=8, D=128, out=16, od=_native.OUT_F32, os_=4096, oh=128, ws=None, wsb=0)
