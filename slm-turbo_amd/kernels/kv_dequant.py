@@ -504,7 +504,8 @@ def kv_dequant_chunk_paged(
                         the kernel, no host sync)
         max_seq_len     the longest of seq_lens, or more
         out, out_dtype  as in kv_dequant_decode_paged_batched
-    Tokens that see no key produce zeros.
+    Tokens that see no key produce zeros; those past query_start_loc[R] belong to no
+    request, and ``out`` keeps what it held there (a new one holds zeros).
     """
     assert q.dim() == 3, f"q must be [N, H, D], got {tuple(q.shape)}"
     N, H, D = q.shape
@@ -530,7 +531,7 @@ def kv_dequant_chunk_paged(
     dev = q.device
     with _on_device(dev):
         if out is None:
-            out = torch.empty((N, H, D), dtype=out_dtype or torch.float32, device=dev)
+            out = torch.zeros((N, H, D), dtype=out_dtype or torch.float32, device=dev)
         out_dtype = out.dtype
         out_stride = out.stride()
         if not ((out_dtype is torch.float32 or out_dtype is torch.float16) and out.shape == (N, H, D)

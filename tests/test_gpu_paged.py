@@ -396,3 +396,22 @@ def test_chunk_slots_past_a_position_stay_out():
         out = out.cpu().numpy()
         assert_close(out[:20], ref[:20], atol=1e-5 * np.abs(ref).max(), rtol=0, what="before the NaNs")
         assert np.isnan(out[20:]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("most", [50, 5000])                              # one part, and several
+def test_chunk_rows_of_no_request(most):
+    """Rows past the last request's: left alone in a given tensor, zeros in a new one."""
+    kd = _kd()
+    dev = "cuda:0"
+    case = make_paged_case(seed=3, B=2, H=8, KV=2, D=64, lens=[40, 50])
+    q = torch.randn(12, 8, 64, generator=torch.Generator().manual_seed(1)).half().to(dev)
+    args = (torch.from_numpy(case.kv_cache).to(dev), case.block_tables.to(dev), case.seq_lens.to(dev),
+            torch.tensor([0, 4, 10], dtype=torch.int32, device=dev), most, 16, 2)
+    given = torch.full((12, 8, 64), 7.0, device=dev)
+    kd.kv_dequant_chunk_paged(q, *args, out=given)
+    assert (given[10:] == 7).all() and not (given[:10] == 7).any()
+    held = [torch.full((12, 8, 64), 7.0, device=dev) for _ in range(4)]     # memory that a new tensor gets again
+    del held
+    new = kd.kv_dequant_chunk_paged(q, *args)
+    assert (new[10:] == 0).all() and torch.equal(new[:10], given[:10])
