@@ -367,3 +367,44 @@ def test_backend_first_chunks_and_short_continuation_match_oracle():
     tokens by 2 new ones in one step: each request attends to its own tokens
     only."""
     _mixed_step_matches_oracle([10, 8, 5], [10, 2, 5], seed=93)
+
+
+# Both routes of a multi-token step, by block size and by few tokens on long contexts,
+# with metadata padded past the requests (as captured steps pad it) and without.
+@pytest.mark.gpu
+@pytest.mark.parametrize("bs,lens,qlens,pad,route", [
+    (16, [307, 1012, 90], [7, 12, 1], True, "kv_dequant_chunk_paged"),
+    (8, [307, 1012, 90], [7, 12, 1], False, "kv_dequant_decode_paged_batched"),
+    (8, [33, 64, 5], [30, 1, 5], True, "kv_dequant_decode_paged_batched"),
+    (16, [40000, 500, 29000], [2, 2, 2], True, "kv_dequant_decode_paged_batched")])
+def test_backend_mixed_step_routes_and_padded_metadata(bs, lens, qlens, pad, route):
+    from kernels import kv_dequant
+
+    H, KV, D, N, R = 8, 2, 128, sum(qlens), len(lens)
+    case = make_paged_case(seed=N, B=R, H=H, KV=KV, D=D, lens=lens, block_size=bs)
+    q = torch.randn(N, H, D, generator=torch.Generator().manual_seed(N)).half()
+    rows = torch.stack([case.block_tables[r] for r, n in enumerate(qlens) for _ in range(n)])
+    vlens = [L - n + i + 1 for L, n in zip(lens, qlens) for i in range(n)]
+    ref = paged_reference(type(case)(q=q, kv_cache=case.kv_cache, block_tables=rows, block_size=bs, num_kv_heads=KV,
+                                     seq_lens=torch.tensor(vlens, dtype=torch.int32)))
+    meta = _chunk_meta(lens, qlens, case.block_tables)
+    if pad:                                   # three requests without tokens, one of them without a length
+        meta.query_start_loc = torch.cat([meta.query_start_loc, torch.full((3,), N, dtype=torch.int32)])
+        meta.seq_lens = torch.cat([meta.seq_lens, torch.tensor([0, 7], dtype=torch.int32)])
+        meta.block_table = torch.cat([meta.block_table, torch.zeros_like(meta.block_table[:1])])
+    dev = "cuda:0"
+    for f in ("seq_lens", "block_table", "query_start_loc"):
+        setattr(meta, f, getattr(meta, f).to(dev))
+    calls = []
+
+    class Seen:
+        def __getattr__(self, name):
+            calls.append(name)
+            return getattr(kv_dequant, name)
+
+    out = torch.full((N + 2, H * D), 3.0, dtype=torch.float16, device=dev)
+    _impl(H=H, D=D, KV=KV, kernels=Seen()).forward(None, q.to(dev), q.to(dev), q.to(dev),
+                                                   torch.from_numpy(case.kv_cache).to(dev), meta, out)
+    assert calls == [route]
+    assert_close(out[:N].float().cpu().numpy().reshape(N, H, D), ref, what="mixed step")
+    assert (out[N:] == 3).all()
