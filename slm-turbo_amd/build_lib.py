@@ -6,8 +6,8 @@
 Each .hip translation unit is compiled to an object in slm-turbo_amd/_build/
 and the objects are linked into slm-turbo_amd/kernels/libslmturbo_hip.so,
 which kernels/kv_dequant.py loads through ctypes.  csrc/pyfast.c becomes the
-CPython module kernels/_slmt_fast (gcc), a low-overhead binding of the two
-per-layer entry points of that same library.
+CPython module kernels/_slmt_fast (gcc), a low-overhead binding of the hot
+entry points of that same library.
 """
 from __future__ import annotations
 

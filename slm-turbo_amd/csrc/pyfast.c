@@ -24,8 +24,16 @@ static int take(PyObject* const* args, Py_ssize_t n, long long* v) {
 #define I(i) ((int)v[i])
 #define L(i) ((int64_t)v[i])
 
-/* One function: N integer arguments, handed on as the entry point's own types. */
-#define ENTRY(name, N, ...)                                                        \
+/*
+ * One function: N integer arguments, handed on as the entry point's own types.  Other
+ * Python threads run meanwhile, as during a ctypes call (a first launch loads code, and
+ * one on a full queue waits), where RUN is FREE.  The decodes keep the lock (HELD): they
+ * share the stream's workspace, which the batched one fills in one launch and reads in
+ * the next, and another thread's decode must not come between these.
+ */
+#define HELD(...) __VA_ARGS__
+#define FREE(...) Py_BEGIN_ALLOW_THREADS __VA_ARGS__ Py_END_ALLOW_THREADS
+#define ENTRY(name, RUN, N, ...)                                                   \
   static __typeof__(slmt_##name)* g_##name = NULL;                                 \
   static PyObject* name(PyObject* self, PyObject* const* args, Py_ssize_t n) {     \
     (void)self;                                                                    \
@@ -39,23 +47,25 @@ static int take(PyObject* const* args, Py_ssize_t n, long long* v) {
       return NULL;                                                                 \
     }                                                                              \
     if (take(args, N, v)) return NULL;                                             \
-    return PyLong_FromLongLong(g_##name(__VA_ARGS__));                             \
+    long long rc;                                                                  \
+    RUN(rc = g_##name(__VA_ARGS__);)                                               \
+    return PyLong_FromLongLong(rc);                                                \
   }
 
-ENTRY(quantize_store, 12, P(0), L(1), P(2), L(3), P(4), L(5), I(6), P(7), L(8), I(9), I(10), P(11))
-ENTRY(decode_paged_batched, 22, P(0), L(1), L(2), P(3), L(4), I(5), P(6), I(7), L(8), P(9), I(10), I(11),
+ENTRY(quantize_store, HELD, 12, P(0), L(1), P(2), L(3), P(4), L(5), I(6), P(7), L(8), I(9), I(10), P(11))
+ENTRY(decode_paged_batched, HELD, 22, P(0), L(1), L(2), P(3), L(4), I(5), P(6), I(7), L(8), P(9), I(10), I(11),
       I(12), I(13), I(14), P(15), I(16), L(17), L(18), P(19), L(20), P(21))
-ENTRY(chunk_paged, 24, P(0), L(1), L(2), P(3), L(4), I(5), P(6), I(7), L(8), P(9), P(10), I(11), I(12), I(13),
+ENTRY(chunk_paged, FREE, 24, P(0), L(1), L(2), P(3), L(4), I(5), P(6), I(7), L(8), P(9), P(10), I(11), I(12), I(13),
       I(14), I(15), I(16), P(17), I(18), L(19), L(20), P(21), L(22), P(23))
-ENTRY(chunk_workspace_bytes, 6, L(0), I(1), I(2), I(3), I(4), I(5))
-ENTRY(decode_per_token, 17, P(0), P(1), P(2), P(3), P(4), P(5), P(6), I(7), I(8), I(9), I(10), I(11), I(12),
+ENTRY(chunk_workspace_bytes, HELD, 6, L(0), I(1), I(2), I(3), I(4), I(5))
+ENTRY(decode_per_token, HELD, 17, P(0), P(1), P(2), P(3), P(4), P(5), P(6), I(7), I(8), I(9), I(10), I(11), I(12),
       P(13), P(14), L(15), P(16))
-ENTRY(decode_per_channel, 18, P(0), P(1), P(2), P(3), P(4), P(5), P(6), I(7), I(8), I(9), I(10), I(11), I(12),
+ENTRY(decode_per_channel, HELD, 18, P(0), P(1), P(2), P(3), P(4), P(5), P(6), I(7), I(8), I(9), I(10), I(11), I(12),
       I(13), P(14), P(15), L(16), P(17))
-ENTRY(prefill_per_channel, 21, P(0), P(1), P(2), P(3), P(4), P(5), P(6), I(7), I(8), I(9), I(10), I(11),
+ENTRY(prefill_per_channel, FREE, 21, P(0), P(1), P(2), P(3), P(4), P(5), P(6), I(7), I(8), I(9), I(10), I(11),
       I(12), I(13), I(14), I(15), I(16), P(17), P(18), L(19), P(20))
-ENTRY(quantize_kv_per_channel, 12, P(0), P(1), I(2), I(3), I(4), P(5), P(6), P(7), P(8), P(9), P(10), P(11))
-ENTRY(quantize_with_rulers, 12, P(0), L(1), L(2), I(3), I(4), I(5), P(6), P(7), P(8), L(9), L(10), P(11))
+ENTRY(quantize_kv_per_channel, FREE, 12, P(0), P(1), I(2), I(3), I(4), P(5), P(6), P(7), P(8), P(9), P(10), P(11))
+ENTRY(quantize_with_rulers, FREE, 12, P(0), L(1), L(2), I(3), I(4), I(5), P(6), P(7), P(8), L(9), L(10), P(11))
 
 /* bind(name, address): the library's entry point slmt_<name> */
 static PyObject* bind(PyObject* self, PyObject* const* args, Py_ssize_t n) {

@@ -201,3 +201,26 @@ def test_fastcall_store_reaches_the_same_checks(lib):
         f.quantize_store("x", 1024, 16, 1024, 16, 4, 16, 16, 1, 8, 128, 0)
     with pytest.raises(TypeError):
         f.decode_paged_batched(*range(21))
+
+
+@pytest.mark.parametrize("name", ["chunk_paged", "prefill_per_channel", "quantize_kv_per_channel", "quantize_with_rulers"])
+def test_fastcall_lets_other_threads_run(lib, name):
+    """As ctypes did: the entry is bound to libc's usleep, and another thread runs while it
+    sleeps.  (The decodes keep the lock: they share a workspace between launches.)"""
+    import threading
+    import time
+
+    f = _fast(lib)
+    usleep = ctypes.CDLL(None).usleep
+    args = len(_native.SIGNATURES["slmt_" + name][1])
+    woke = []
+    f.bind(name, ctypes.cast(usleep, ctypes.c_void_p).value)
+    try:
+        t = threading.Thread(target=lambda: (time.sleep(0.02), woke.append(time.monotonic())))
+        t.start()
+        assert getattr(f, name)(400_000, *[0] * (args - 1)) == 0
+        done = time.monotonic()
+        t.join()
+    finally:
+        f.bind(name, ctypes.cast(getattr(lib, "slmt_" + name), ctypes.c_void_p).value)
+    assert woke[0] < done - 0.1
