@@ -129,7 +129,10 @@ __device__ __forceinline__ uint32_t nib_pair(uint32_t lo_all, uint32_t hi_all, i
 // rows): the K/V tiles are staged once, by the first four waves, for all of them.
 // Head_dim 64 is held to 128 VGPRs, four waves per SIMD (two 8-wave workgroups
 // per CU).
-template <int D, int HP>
+// BIG: a KV head's codes are 2^32 bytes or more, and a tile's place in them is added to
+// the base (with every call that way the addresses spilled 30 to 100 registers at head_dim
+// 64, 13 %).
+template <int D, int HP, bool BIG>
 __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : D == 80 ? 2 : 1))) prefill_kernel(const Params p) {
   using GG = Geo<D>;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -240,8 +243,8 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
       }
   }
   // The KV head's code planes from scalar registers, the lane's place in them as
-  // 32-bit offsets (a plane is S * D / 2 < 2^32 bytes): scalar base plus vector
-  // offset loads, and no 64-bit per-lane pointers held across the loop.
+  // 32-bit offsets (a plane is S * D / 2 < 2^32 bytes, but for BIG): scalar base plus
+  // vector offset loads, and no 64-bit per-lane pointers held across the loop.
   const int kvs = __builtin_amdgcn_readfirstlane(kv);
   const uint8_t* const kbase = p.kp + (int64_t)kvs * p.S * (D / 2);
   const uint8_t* const vbase = p.vp + (int64_t)kvs * p.S * (D / 2);
@@ -255,36 +258,39 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
   auto load = [&](int t, auto slot) {   // the tile's codes (keys past S re-read key S - 1)
     constexpr int sl = decltype(slot)::value;
     if (!stager) return;
+    const uint8_t* const kt = BIG ? kbase + (int64_t)t * (BN * (D / 2)) : kbase;
+    const uint8_t* const vt = BIG ? vbase + (int64_t)t * (BN * (D / 2)) : vbase;
     if ((t + 1) * BN <= p.S) {             // uniform: every key of the tile lies before S
-      const uint32_t off = (uint32_t)t * BN * (D / 2);
+      const uint32_t off = BIG ? 0 : (uint32_t)t * BN * (D / 2);
 #pragma unroll
-      for (int i = 0; i < GG::KW; ++i) kx[sl][i] = *reinterpret_cast<const uint2*>(kbase + (koff0 + off + 8 * i));
+      for (int i = 0; i < GG::KW; ++i) kx[sl][i] = *reinterpret_cast<const uint2*>(kt + (koff0 + off + 8 * i));
 #pragma unroll
       for (int r = 0; r < GG::VW; ++r) {
-        vx[sl][r][0] = *reinterpret_cast<const uint32_t*>(vbase + (voff0 + off + 32 * r));
-        vx[sl][r][1] = *reinterpret_cast<const uint32_t*>(vbase + (voff0 + off + D / 2 + 32 * r));
+        vx[sl][r][0] = *reinterpret_cast<const uint32_t*>(vt + (voff0 + off + 32 * r));
+        vx[sl][r][1] = *reinterpret_cast<const uint32_t*>(vt + (voff0 + off + D / 2 + 32 * r));
       }
       if constexpr (GG::X) {
-        kxx[sl] = *reinterpret_cast<const uint16_t*>(kbase + (koff0 + off + 32 - 6 * ku));
-        vxx[sl][0] = vbase[voff0 + off + 32 - 3 * vb];
-        vxx[sl][1] = vbase[voff0 + off + D / 2 + 32 - 3 * vb];
+        kxx[sl] = *reinterpret_cast<const uint16_t*>(kt + (koff0 + off + 32 - 6 * ku));
+        vxx[sl][0] = vt[voff0 + off + 32 - 3 * vb];
+        vxx[sl][1] = vt[voff0 + off + D / 2 + 32 - 3 * vb];
       }
       return;
     }
-    const int key = min(t * BN + kk, p.S - 1);
+    const int lead = BIG ? t * BN : 0;
+    const int key = min(t * BN + kk, p.S - 1) - lead;
     const uint32_t ko = (uint32_t)(key * (D / 2) + ku * 8 * GG::KW);
 #pragma unroll
-    for (int i = 0; i < GG::KW; ++i) kx[sl][i] = *reinterpret_cast<const uint2*>(kbase + (ko + 8 * i));
-    const int k0 = min(t * BN + 2 * vk, p.S - 1), k1 = min(t * BN + 2 * vk + 1, p.S - 1);
+    for (int i = 0; i < GG::KW; ++i) kx[sl][i] = *reinterpret_cast<const uint2*>(kt + (ko + 8 * i));
+    const int k0 = min(t * BN + 2 * vk, p.S - 1) - lead, k1 = min(t * BN + 2 * vk + 1, p.S - 1) - lead;
 #pragma unroll
     for (int r = 0; r < GG::VW; ++r) {
-      vx[sl][r][0] = *reinterpret_cast<const uint32_t*>(vbase + (uint32_t)(k0 * (D / 2) + 4 * (vb + 8 * r)));
-      vx[sl][r][1] = *reinterpret_cast<const uint32_t*>(vbase + (uint32_t)(k1 * (D / 2) + 4 * (vb + 8 * r)));
+      vx[sl][r][0] = *reinterpret_cast<const uint32_t*>(vt + (uint32_t)(k0 * (D / 2) + 4 * (vb + 8 * r)));
+      vx[sl][r][1] = *reinterpret_cast<const uint32_t*>(vt + (uint32_t)(k1 * (D / 2) + 4 * (vb + 8 * r)));
     }
     if constexpr (GG::X) {
-      kxx[sl] = *reinterpret_cast<const uint16_t*>(kbase + (ko + 32 - 6 * ku));
-      vxx[sl][0] = vbase[(uint32_t)(k0 * (D / 2) + 32 + vb)];
-      vxx[sl][1] = vbase[(uint32_t)(k1 * (D / 2) + 32 + vb)];
+      kxx[sl] = *reinterpret_cast<const uint16_t*>(kt + (ko + 32 - 6 * ku));
+      vxx[sl][0] = vt[(uint32_t)(k0 * (D / 2) + 32 + vb)];
+      vxx[sl][1] = vt[(uint32_t)(k1 * (D / 2) + 32 + vb)];
     }
   };
   auto store = [&](auto slot) {  // slot's codes -> fp16 (code - zero) in LDS stage `slot`
@@ -575,17 +581,17 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
   }
 }
 
-template <int D, int HP>
+template <int D, int HP, bool BIG = false>
 int launch_hp(Params p, hipStream_t stream) {
   static const bool lds_ok = [] {   // above 64 KB of LDS (head_dim 128) needs the attribute
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_kernel<D, HP>),
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_kernel<D, HP, BIG>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, Geo<D>::LDS + 1024 * HP) == hipSuccess;
   }();
   if (!lds_ok) return fail(SLMT_ERR_HIP, "prefill: could not grant the kernel its LDS");
   const int grid = p.qblocks * (p.H / HP);
   const int cus = device_cu_count();
   p.paired = HP == 1 && p.causal && 8 * grid >= 11 * cus && grid <= 2 * cus;
-  hipLaunchKernelGGL((prefill_kernel<D, HP>), dim3(grid), dim3(256 * HP), Geo<D>::LDS + 1024 * HP, stream, p);
+  hipLaunchKernelGGL((prefill_kernel<D, HP, BIG>), dim3(grid), dim3(256 * HP), Geo<D>::LDS + 1024 * HP, stream, p);
   return check_launch("prefill");
 }
 
@@ -599,6 +605,7 @@ int launch_hp(Params p, hipStream_t stream) {
 // rounds the longest must start first (+16 to 23 %).
 template <int D>
 int launch(const Params& p, hipStream_t stream) {
+  if ((int64_t)p.S * (D / 2) >= int64_t(1) << 32) return launch_hp<D, 1, true>(p, stream);
   if (p.G % 2 == 0 && (int64_t)p.qblocks * (p.H / 2) > 256) return launch_hp<D, 2>(p, stream);
   return launch_hp<D, 1>(p, stream);
 }

@@ -480,3 +480,17 @@ def test_head_dim_80_zero_points_that_are_no_numbers(bad):
         assert_close(out[H // KV:], ref[H // KV:], what=f"zero point {bad}, the other KV head")
     raw = _kd().kv_dequant_decode_attention(q.to(DEV), *dev, use_quant=False)
     assert torch.isfinite(raw).all()                                     # the raw codes need no ruler
+
+
+def test_prefill_codes_past_four_gib():
+    """A KV head's codes pass 2^32 bytes: the last keys, which take all of the weight, are
+    read where they lie and not from the start."""
+    D, S = 80, 2**32 // 40 + 300
+    q = torch.ones(1, 1, D, dtype=torch.float16, device=DEV)
+    one, zero = torch.ones(1, D, dtype=torch.float16, device=DEV), torch.zeros(1, D, dtype=torch.float16, device=DEV)
+    k = torch.zeros(1, S, D // 2, dtype=torch.uint8, device=DEV)
+    v = torch.zeros_like(k)
+    k[:, -100:] = 0xFF
+    v[:, -100:] = 0x33
+    out = _kd().kv_dequant_prefill_attention(q, k, one, zero, v, one, zero, causal=False)
+    assert (out - 3.0).abs().max() <= 1e-5                                   # exp(-134) for every other key
