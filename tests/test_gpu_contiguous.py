@@ -362,8 +362,8 @@ def test_decode_per_channel_split_chunks(H, KV, D, S, outl):
         assert_close(out.cpu().numpy(), ref, what=f"H={H} KV={KV} D={D} S={S}")
 
 
-# The register kernel's thread and row counts (up to 4096 rows), the three launches
-# past it (chunks with remainders, several KV heads), inputs at odd multiples of 4
+# The register kernel's thread and row counts (up to 8192 rows), the three launches
+# past it (test_quantize_kv_long has more of these), inputs at odd multiples of 4
 # bytes, NaN and infinities, constant channels: each byte against the oracle, K and
 # V together as one by one.
 @pytest.mark.parametrize("KV,S,D", [(1, 1, 64), (2, 31, 80), (3, 32, 128), (2, 33, 64), (1, 511, 80), (2, 513, 128),
@@ -383,6 +383,34 @@ def test_quantize_kv_row_counts(KV, S, D):
     got = _kd().quantize_kv(kd_, v.to(DEV))
     alone = _kd().quantize_per_channel(kd_)
     torch.cuda.synchronize()
+    ref = oq.quantize_kv(k.numpy(), v.numpy())
+    for i, (a, b) in enumerate(zip(got, ref)):
+        if a.dtype == torch.uint8:
+            assert np.array_equal(a.cpu().numpy(), b), f"codes {i}: {int((a.cpu().numpy() != b).sum())} differ"
+        else:
+            _same_fp16(a.cpu().numpy(), b)
+    for a, b in zip(alone, got):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+# The last register case and the three launches: every head_dim (80: 25 rows a pass and 6
+# idle threads), several KV heads (whose minima and maxima wait in their own codes), chunk
+# counts held down by the KV heads, remainders, and special values in the last row of the
+# last chunk of the last KV head.
+@pytest.mark.parametrize("KV,S,D", [(1, 8192, 64), (2, 8193, 64), (2, 8193, 80), (3, 9001, 128), (2, 20011, 80),
+                                    (40, 8200, 80), (1, 70001, 128)])
+def test_quantize_kv_long(KV, S, D):
+    g = torch.Generator().manual_seed(S + D)
+    k, v = torch.randn(KV, S, D, generator=g).half(), (3 * torch.randn(KV, S, D, generator=g)).half()
+    k[KV - 1, S - 1, D - 1] = float("nan")
+    k[KV - 1, S - 1, D - 2] = float("inf")
+    k[KV - 1, S - 1, 0] = -60000.0
+    k[0, 0, 1] = 500.0
+    v[KV - 1, :, 4] = 0.25
+    v[KV - 1, S - 1, D - 1] = 100.0
+    v[KV - 1, S // 2, 3] = -float("inf")
+    got = _kd().quantize_kv(k.to(DEV), v.to(DEV))
+    alone = _kd().quantize_per_channel(k.to(DEV))
     ref = oq.quantize_kv(k.numpy(), v.numpy())
     for i, (a, b) in enumerate(zip(got, ref)):
         if a.dtype == torch.uint8:
