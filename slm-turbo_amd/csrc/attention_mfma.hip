@@ -60,7 +60,10 @@
 // weight loses precision below 2^-14 and vanishes below 2^-25: a long tail
 // behind a dominant token would drop out).  The pair is joined once per
 // segment; the softmax sums use p itself, and the per-token min enters once per
-// token as sum(p * min).
+// token as sum(p * min).  fp32 output is 1.3e-5 off 64 bits, from the subnormal codes: a
+// full-precision weight times one loses up to 10 bits in the matrix core (with all codes
+// 1 the error is 9e-6 of sum(p n), with random codes 1e-6, with q = 0, where every weight
+// is a power of two times its step, 3e-8).
 #include "attention_kernel.h"
 
 #include <hip/hip_ext.h>

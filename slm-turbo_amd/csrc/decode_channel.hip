@@ -32,7 +32,7 @@
 // and sum(p * V min) joins both dims of every lane.  All in fp32; the general
 // kernel, which served these calls and head_dim 80 before, holds its weights in 16
 // bits and walks 16-token tiles through two barriers each: 3000 tokens, 32 q / 8 KV
-// heads, 128 dims 47.4 -> 11.5 us per call (the host's part is 10).
+// heads, 128 dims 47.4 -> 11.5 us per call (the host's part is 7.5).
 // use_quant = 0 attends over the raw codes.  Keys are loaded once, coalesced
 // (4 lanes per key row); V rows are staged in LDS for the byte-wise PV.
 #include "attention_kernel.h"

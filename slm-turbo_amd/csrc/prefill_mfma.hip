@@ -53,8 +53,8 @@
 // dim 63 are staged evenly too, 2 bytes of K and 1 byte of V per key and thread,
 // so that no wave has more to convert than another.  Against the vector-ALU
 // kernel that took one query row at a time, us per causal prefill: 32 q / 8 KV
-// heads, 1000 tokens 481 -> 25, 4096 tokens 6277 -> 180; 8/8, 100 tokens 32.6 ->
-// 8.5 (the call's host time).  186 VGPRs, two waves per SIMD.
+// heads, 1000 tokens 481 -> 24, 4096 tokens 6277 -> 184; 8/8, 100 tokens 32.6 ->
+// 8.5 (the call's host time).  212 to 218 VGPRs, two waves per SIMD.
 #include "slmt_internal.h"
 
 #include <type_traits>
@@ -535,7 +535,7 @@ __global__ void __launch_bounds__(256 * HP) __attribute__((amdgpu_waves_per_eu(D
   using T = std::true_type;
   using F = std::false_type;
   if (HP == 1 || stager) wide ? run(T{}, T{}) : run(T{}, F{});
-  else wide ? run(F{}, T{}) : run(F{}, F{});
+  else wide ? run(F{}, T{}) : run(F{}, F{});   // (head_dim 64 spills registers in the wide loops alone)
 
   // every row of the ones product holds the column's whole sum
   const float rl = 1.0f / ol[0];

@@ -214,7 +214,7 @@ struct AttnParams {
   const int32_t* seq_lens;
   int fixed_len;
   int B, H, G;           // G = H / num_kv_heads
-  int heads_per_group;   // query heads per workgroup (multiple of 4)
+  int heads_per_group;   // query heads per workgroup (a multiple of 4 but on the matrix cores)
   // output: element (b, h, d) at out + b*out_seq_stride + h*out_head_stride + d
   void* out;
   int out_f16;
@@ -234,8 +234,8 @@ struct AttnPlan {
   int heads_per_group, groups, waves, W, W_ws;
   bool dma;
   size_t lds_bytes;
-  // whole-row kernel (head_dim 128, 4 or 8 query heads per KV head): KV heads
-  // and waves per KV head of a workgroup, head groups
+  // whole-row kernels (attention_mfma.hip, attention_rows.hip): KV heads and waves per
+  // KV head of a workgroup, head groups
   bool rows, mfma;   // mfma: the matrix-core kernel of the two
   int rows_nkv, rows_wpk, rows_groups;
 };
@@ -302,7 +302,8 @@ struct ChunkParams {
 int64_t chunk_workspace_bytes(int64_t N, int R, int H, int KV, int D, int max_seq_len);
 int launch_chunk(int D, ChunkParams& p, int max_seq_len, void* workspace, int64_t ws_bytes, hipStream_t stream);
 
-// Per-channel prefill on the matrix cores (prefill_mfma.hip); no workspace.  q [H, M, D] fp16, codes [KV_t, S, D/2], rulers [KV_t, D].
+// Per-channel prefill on the matrix cores (prefill_mfma.hip); no workspace.  q [H, M, D]
+// fp16, codes [KV_t, S, D/2], rulers [KV_t, D].
 int launch_prefill_mfma(const void* q, const void* kp, const void* ks, const void* kz, const void* vp, const void* vs,
                         const void* vz, int H, int G, int M, int S, int D, int causal, int use_quant, float* out,
                         hipStream_t stream);
