@@ -522,3 +522,26 @@ def test_prefill_codes_past_four_gib():
     v[:, -100:] = 0x33
     out = _kd().kv_dequant_prefill_attention(q, k, one, zero, v, one, zero, causal=False)
     assert (out - 3.0).abs().max() <= 1e-5                                   # exp(-134) for every other key
+
+
+@pytest.mark.parametrize("H,KV,D", [(32, 8, 64), (32, 4, 80), (32, 8, 128)])
+def test_prefill_wide_range_queries_two_heads_per_workgroup(H, KV, D):
+    """The long prefills' form (more than 256 workgroups of two heads): waves with and
+    without such columns, staging and not, walk different loops through the same barriers."""
+    M = 1100
+    g = torch.Generator().manual_seed(D)
+    q = torch.randn(H, M, D, generator=g)
+    q[:, 5::97] *= 1e4
+    q[1::2, 200:300] *= 1e4
+    q = q.clamp(-65504, 65504).half()
+    packed = torch.randint(0, 256, (2, KV, M, D // 2), generator=g, dtype=torch.uint8)
+    scale = (torch.rand(2, KV, D, generator=g) * 0.4 + 0.05).half()
+    scale[0, 0] *= 500
+    zero = torch.randint(0, 16, (2, KV, D), generator=g).half()
+    t = (packed[0], scale[0], zero[0], packed[1], scale[1], zero[1])
+    out = _kd().kv_dequant_prefill_attention(q.to(DEV), *[x.to(DEV) for x in t]).cpu()
+    G, heads = H // KV, [0, 1, H // KV, H - 1]
+    for h in heads:
+        one = [x[h // G: h // G + 1].numpy() for x in t]
+        assert_close(out[h:h + 1].numpy(), oa.prefill_per_channel(q[h:h + 1].numpy(), *one), what=f"D={D} head {h}")
+    assert torch.isfinite(out).all()
